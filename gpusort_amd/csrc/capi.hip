@@ -145,7 +145,7 @@ gs_status sort_device(gs_handle* h, gs_dtype kdt, void* d_keys, gs_dtype vdt, vo
   const int vb = val_bytes_of(vdt);
   const XformParams xf = make_xform((int)kdt, descending != 0);
   if (n <= 1) return GS_OK;
-  if (n <= block_sort_max(kb, vb)) {
+  if (n <= block_sort_tile_max(kb, vb)) {
     return from_hip(block_sort(kb, vb, d_keys, d_vals, (uint32_t)n, xf, h->stream), "block sort");
   }
   const size_t ws_bytes = radix_workspace_bytes(kb, vb, n);

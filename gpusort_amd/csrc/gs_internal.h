@@ -103,9 +103,10 @@ hipError_t multisplit(int key_bytes, int val_bytes, const void* keys, const void
 uint32_t radix_seg_tile_keys(int key_bytes, int val_bytes, int geo);
 
 // Size classes of the batched segmented sort: segments of at most small_max
-// keys (<= block_sort_max) are sorted by the LDS bitonic kernel, those of at
-// most medium_max by the segmented onesweep with the small tiles, the rest
-// with the large tiles.
+// keys (<= block_sort_max) are sorted in LDS, those of at
+// most medium_max by the segmented onesweep with the small tiles, the rest in
+// LDS where they fit one tile (block_sort_tile_max) and with the large tiles
+// where not.
 struct SegConfig {
   uint32_t small_max;
   uint64_t medium_max;
@@ -120,21 +121,23 @@ hipError_t radix_sort_segments(int key_bytes, int val_bytes, void* keys, void* v
                                LaunchTimer* timer = nullptr, int tile_policy = kTilesByStream);
 
 // ---------------------------------------------------------------- block sort
-// Single-workgroup stable sort of n <= block_sort_max(key_bytes, val_bytes)
-// keys held in LDS (bitonic network over (key, original index) pairs).
+// Single-workgroup stable sort of n <= block_sort_tile_max(key_bytes,
+// val_bytes) keys held in LDS.  block_sort_max is the largest small-segment
+// limit a size-class configuration may set.
 uint32_t block_sort_max(int key_bytes, int val_bytes);
+uint32_t block_sort_tile_max(int key_bytes, int val_bytes);
 hipError_t block_sort(int key_bytes, int val_bytes, void* keys, void* vals, uint32_t n, const XformParams& xf,
                       hipStream_t stream);
 
 // Batched variant: workgroup b sorts segment s = d_seg_ids[b] (or b when
-// d_seg_ids is null), i.e. keys[off[s] .. off[s+1]), which must be no longer
-// than block_sort_max.  max_len (0: unknown) bounds the segments' length;
-// up to kBlockSortSmall keys a smaller workgroup with a smaller LDS tile is
-// used, so more of them share a CU.
-constexpr uint32_t kBlockSortSmall = 1024;
+// d_seg_ids is null), i.e. keys[off[s] .. off[s+1]).  One launch takes
+// segments of one length class (block_sort_class of each: the workgroup and
+// its LDS tile grow with the class); longer ones are left untouched.
+constexpr int kBlockClasses = 5;
+int block_sort_class(int key_bytes, int val_bytes, uint32_t len);
 hipError_t block_sort_segments(int key_bytes, int val_bytes, void* keys, void* vals, const uint64_t* d_offsets,
                                const uint32_t* d_seg_ids, uint32_t nblocks, const XformParams& xf,
-                               hipStream_t stream, uint32_t max_len = 0);
+                               hipStream_t stream, int cls);
 
 // ---------------------------------------------------------------- merge path
 // One 2-way merge job: out[out_off ..) = merge(a[a_off, a_off+a_len), b[b_off, b_off+b_len)),

@@ -5,8 +5,8 @@
 // sequence and one synchronisation per array.  Here every segment of one
 // call is sorted by a fixed number of launches, whatever the count:
 //
-//   small  (<= one LDS tile, block_sort_max): one workgroup per segment,
-//          bitonic network in LDS, all small segments in one launch
+//   small  (<= one LDS tile): one workgroup per segment, sorted in LDS
+//          (block_sort.hip), one launch per length class
 //   radix  (up to 2^30 keys): segmented onesweep -- one histogram launch,
 //          one scan launch and one launch per digit for all of them; tiles
 //          never straddle segments and the look-back stops at the segment's
@@ -40,15 +40,15 @@ struct SegPlanHost {
   int kb = 4, vb = 0;
   uint32_t nseg = 0;
   uint64_t n_total = 0;
-  std::vector<uint32_t> small_ids, multi_ids[2], single_ids[2], huge;
-  uint32_t small_len = 0;  // longest segment of the LDS class
+  // LDS classes by length (block_sort_class), radix groups, single-array sorts.
+  std::vector<uint32_t> small_ids[kBlockClasses], multi_ids[2], single_ids[2], huge;
   struct Group {
     int geo = 0;  // tile geometry (radix_seg_tile_keys)
     uint32_t nslots = 0;
     uint64_t tiles = 0, n_keys = 0, tile_keys = 0;
     size_t off_tile_seg = 0, off_seg_first = 0, off_seg_range = 0;
   } grp[2];
-  size_t off_small = 0, off_offsets = 0;
+  size_t off_small[kBlockClasses] = {}, off_offsets = 0;
   std::vector<unsigned char> meta;
   size_t ws_bytes = 0;  // workspace of the radix groups
 };
@@ -62,14 +62,17 @@ void build_seg_plan(int kb, int vb, const uint64_t* off, uint32_t nseg, const Se
   P->nseg = nseg;
   P->n_total = off[nseg];
   const uint32_t small_max = std::min<uint32_t>(cfg.small_max, block_sort_max(kb, vb));
+  // A segment past the medium class that fits one LDS tile is read and
+  // written once there instead of once per digit: 4300 arrays of 4097-16384
+  // pairs 0.41 ms, as part of the large-tile passes about 0.9 ms.
+  const uint64_t tile_max = block_sort_tile_max(kb, vb);
   P->grp[0].geo = 0;
   P->grp[1].geo = 1 + (int)std::min<uint32_t>(cfg.medium_geometry, 2u);
   for (uint32_t s = 0; s < nseg; ++s) {
     const uint64_t len = off[s + 1] - off[s];
     if (len <= 1) continue;
-    if (len <= small_max) {
-      P->small_ids.push_back(s);
-      P->small_len = std::max(P->small_len, (uint32_t)len);
+    if (len <= small_max || (len > cfg.medium_max && len <= tile_max)) {
+      P->small_ids[block_sort_class(kb, vb, (uint32_t)len)].push_back(s);
     } else if (len >= kSegRadixMax) {
       P->huge.push_back(s);
     } else {
@@ -93,8 +96,10 @@ void build_seg_plan(int kb, int vb, const uint64_t* off, uint32_t nseg, const Se
     if (G.nslots)
       P->ws_bytes = std::max(P->ws_bytes, radix_segments_workspace_bytes(kb, vb, P->n_total, G.tiles, G.nslots));
   }
-  P->off_small = o;
-  o = align_up(o + P->small_ids.size() * 4, 256);
+  for (int c = 0; c < kBlockClasses; ++c) {
+    P->off_small[c] = o;
+    o = align_up(o + P->small_ids[c].size() * 4, 256);
+  }
   P->off_offsets = o;
   o = align_up(o + (size_t)(nseg + 1) * 8, 256);
   P->meta.assign(o, 0);
@@ -119,12 +124,15 @@ void build_seg_plan(int kb, int vb, const uint64_t* off, uint32_t nseg, const Se
       }
     }
   }
-  if (!P->small_ids.empty()) memcpy(b + P->off_small, P->small_ids.data(), P->small_ids.size() * 4);
+  for (int c = 0; c < kBlockClasses; ++c)
+    if (!P->small_ids[c].empty()) memcpy(b + P->off_small[c], P->small_ids[c].data(), P->small_ids[c].size() * 4);
   memcpy(b + P->off_offsets, off, (size_t)(nseg + 1) * 8);
 }
 
 bool seg_plan_empty(const SegPlanHost& P) {
-  return P.small_ids.empty() && P.grp[0].nslots == 0 && P.grp[1].nslots == 0;
+  for (const auto& ids : P.small_ids)
+    if (!ids.empty()) return false;
+  return P.grp[0].nslots == 0 && P.grp[1].nslots == 0;
 }
 
 // Kernel launches only (no copies from host memory, no allocation, no
@@ -133,10 +141,10 @@ hipError_t launch_seg_plan(const SegPlanHost& P, const unsigned char* dm, void* 
                            const XformParams& xf, hipStream_t stream, LaunchTimer* timer,
                            int tile_policy = kTilesByStream) {
   hipError_t e = hipSuccess;
-  if (!P.small_ids.empty()) {
+  for (int c = kBlockClasses - 1; c >= 0; --c) {  // the longest first
     e = block_sort_segments(P.kb, P.vb, d_keys, d_vals, reinterpret_cast<const uint64_t*>(dm + P.off_offsets),
-                            reinterpret_cast<const uint32_t*>(dm + P.off_small), (uint32_t)P.small_ids.size(), xf,
-                            stream, P.small_len);
+                            reinterpret_cast<const uint32_t*>(dm + P.off_small[c]), (uint32_t)P.small_ids[c].size(),
+                            xf, stream, c);
     if (e != hipSuccess) return e;
   }
   for (int g = 1; g >= 0; --g) {

@@ -244,9 +244,10 @@ gs_status gs_profile_begin(gs_handle* h);
 gs_status gs_profile_end(gs_handle* h, gs_kernel_stat* out, uint32_t max_out, uint32_t* n_out);
 
 /* Size classes of the batched sort for one (key, payload) width pair:
- * segments of at most small_max keys (at most the LDS tile) are sorted by the
- * LDS bitonic kernel, those of at most medium_max by the segmented onesweep
- * with small (4K / 3K-key) tiles, the rest with the large tiles.  Kept per
+ * segments of at most small_max keys (at most the LDS tile) are sorted in LDS,
+ * one workgroup each, those of at most medium_max by the segmented onesweep
+ * with small (4K / 3K-key) tiles, the rest in LDS where one workgroup holds
+ * them (up to 9K-16K keys) and with the large tiles where not.  Kept per
  * handle; gs_autotune_segments picks them by measurement.  No counterpart in
  * the reference (one array per call, src/cuda_utils.cu:97-243). */
 typedef struct gs_seg_config {
