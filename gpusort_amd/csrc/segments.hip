@@ -31,6 +31,9 @@ using namespace gs;
 namespace gs {
 
 constexpr uint64_t kSegRadixMax = 1ull << 30;
+// Segments that one launch of the widest LDS class sorts side by side (one
+// workgroup per CU).
+constexpr size_t kOneRound = 256;
 
 SegConfig default_seg_config(int kb, int vb) { return SegConfig{block_sort_max(kb, vb), 0}; }
 
@@ -79,6 +82,17 @@ void build_seg_plan(int kb, int vb, const uint64_t* off, uint32_t nseg, const Se
       const int g = len <= cfg.medium_max ? 1 : 0;
       (len > radix_seg_tile_keys(kb, vb, P->grp[g].geo) ? P->multi_ids[g] : P->single_ids[g]).push_back(s);
     }
+  }
+  // Classes that together leave CUs idle share the launch of the longer one: a
+  // launch lasts as long as its longest segment (4 us for the shortest class,
+  // 40 for the longest), and launches follow one another.
+  for (int c = 0; c + 1 < kBlockClasses; ++c) {
+    int d = c + 1;
+    while (d + 1 < kBlockClasses && P->small_ids[d].empty()) ++d;
+    std::vector<uint32_t>&a = P->small_ids[c], &b = P->small_ids[d];
+    if (a.empty() || b.empty() || a.size() + b.size() > kOneRound) continue;
+    b.insert(b.end(), a.begin(), a.end());
+    a.clear();
   }
   size_t o = 0;
   for (int g = 0; g < 2; ++g) {
