@@ -41,7 +41,15 @@ struct SortCtrl {
   // tiles in XCD groups.
   uint32_t class_counter[kMaxPasses][8];
   uint32_t pad[14];
+  // 64-bit keys (radix_ties.h): the number of highest digits sorted by (0:
+  // all), and the long runs listed for it.  In a cache line without ticket
+  // counters: every workgroup of a segmented pass reads it.
+  uint32_t top_digits;
+  uint32_t long_count;
+  __host__ __device__ uint32_t low() const { return top_digits ? 8u - top_digits : 0u; }
+  uint32_t pad2[30];
 };
+static_assert(sizeof(SortCtrl) == 512, "tickets in the first three 128-byte lines, top_digits in the fourth");
 
 // Optional per-launch timing: when a launcher is given a timer it brackets
 // each kernel with events recorded on the launch stream.  `bytes` is the
@@ -131,8 +139,8 @@ hipError_t block_sort(int key_bytes, int val_bytes, void* keys, void* vals, uint
 
 // Batched variant: workgroup b sorts segment s = d_seg_ids[b] (or b when
 // d_seg_ids is null), i.e. keys[off[s] .. off[s+1]).  One launch takes
-// segments of one length class (block_sort_class of each: the workgroup and
-// its LDS tile grow with the class); longer ones are left untouched.
+// segments of up to one length class (block_sort_class of each: the workgroup
+// and its LDS tile grow with the class); longer ones are left untouched.
 constexpr int kBlockClasses = 5;
 int block_sort_class(int key_bytes, int val_bytes, uint32_t len);
 hipError_t block_sort_segments(int key_bytes, int val_bytes, void* keys, void* vals, const uint64_t* d_offsets,

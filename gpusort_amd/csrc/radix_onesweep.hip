@@ -5,13 +5,15 @@
 //   thrust::sort_by_key  (src/cuda_utils.cu:477-478)   -- stable, with payload
 //
 // One sort is 3 + P launches on one stream, with no host synchronisation:
-//   fill      zero the global digit histograms
+//   prep      zero the global digit histograms; 64-bit keys: pick the lowest
+//             digit to sort by from a sample (radix_ties.h)
 //   hist      one read of all keys -> the 256-bin histogram of every digit
 //             position, and zero of every pass's look-back status words
 //   scan      exclusive digit offsets per pass; passes whose digit is the same
 //             for every key are marked skipped and the ping-pong buffer of
 //             every remaining pass is chosen on the device
 //   pass x P  onesweep pass (below)
+//   ties      64-bit keys: two launches that order what the passes left
 //   copy      only if the result ended in the temporary buffer
 //
 // Onesweep pass, per tile of THREADS*ITEMS keys (tile order from an atomic
@@ -33,6 +35,7 @@
 
 #include "gs_device.h"
 #include "gs_internal.h"
+#include "radix_ties.h"
 
 namespace gs {
 
@@ -71,36 +74,42 @@ struct Vec16<uint64_t> {
 constexpr int kHistThreads = 1024;
 constexpr uint64_t kHistKeysPerThread = 1024;
 
-template <typename U, bool IDENT>
-__global__ __launch_bounds__(kHistThreads) void radix_hist_kernel(const U* __restrict__ keys, uint64_t n, Xform<U> xf,
-                                                                  int passes, unsigned long long* __restrict__ g_hist,
-                                                                  uint4* __restrict__ zero_ptr, uint64_t zero_vec4) {
-  constexpr int MAXP = sizeof(U);  // one 8-bit digit per key byte
-  constexpr uint32_t WORDS = MAXP * (kRadix / 2) * 32;
-  __shared__ __attribute__((aligned(16))) uint32_t s_cnt[WORDS];
+// Only digits from LOW up are counted (LOW even, at most the lowest digit
+// sorted by): the kernel is bound by its LDS adds.
+template <bool IDENT, int LOW>
+__device__ __forceinline__ void radix_hist_from(const uint64_t* __restrict__ keys, uint64_t n, const Xform<uint64_t>& xf,
+                                                unsigned long long* __restrict__ g_hist, uint32_t* s_cnt) {
+  using U = uint64_t;
+  constexpr int MAXP = 8;  // one 8-bit digit per key byte
   const uint32_t tid = threadIdx.x;
   const uint32_t copy = tid & 31u;
   uint4* s4 = reinterpret_cast<uint4*>(s_cnt);
-  for (uint32_t i = tid; i < (uint32_t)passes * (kRadix / 2) * 32 / 4; i += kHistThreads) s4[i] = make_uint4(0, 0, 0, 0);
+  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * (kRadix / 2) * 32 / 4; i += kHistThreads)
+    s4[i] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
   const uint64_t gtid = (uint64_t)blockIdx.x * kHistThreads + tid;
   const uint64_t gstride = (uint64_t)gridDim.x * kHistThreads;
-  for (uint64_t i = gtid; i < zero_vec4; i += gstride) zero_ptr[i] = make_uint4(0, 0, 0, 0);
-  __syncthreads();
-
-  // Every key byte is a pass here (passes == MAXP): the pass offsets are
-  // constants of the unrolled loop.
+  // The digits' offsets are constants of the unrolled loop.
   auto count = [&](U u) {
 #pragma unroll
-    for (int p = 0; p < MAXP; ++p) {
+    for (int p = LOW; p < MAXP; ++p) {
       const uint32_t d = digit_of(u, p * 8);
-      atomicAdd(&s_cnt[p * (kRadix / 2) * 32 + (d >> 1) * 32u + copy], 1u << ((d & 1u) << 4));
+      atomicAdd(&s_cnt[(p - LOW) * (kRadix / 2) * 32 + (d >> 1) * 32u + copy], 1u << ((d & 1u) << 4));
     }
   };
   using VT = typename Vec16<U>::T;
   constexpr int VN = Vec16<U>::N;
   const uint64_t nvec = n / VN;
   const VT* kv = reinterpret_cast<const VT*>(keys);
-  for (uint64_t vi = gtid; vi < nvec; vi += gstride) {
+  uint64_t vi = gtid;
+  for (; vi + gstride < nvec; vi += 2 * gstride) {
+    const VT v = kv[vi], w = kv[vi + gstride];
+#pragma unroll
+    for (int e = 0; e < VN; ++e) count(IDENT ? Vec16<U>::get(v, e) : to_ordered(Vec16<U>::get(v, e), xf));
+#pragma unroll
+    for (int e = 0; e < VN; ++e) count(IDENT ? Vec16<U>::get(w, e) : to_ordered(Vec16<U>::get(w, e), xf));
+  }
+  if (vi < nvec) {
     const VT v = kv[vi];
 #pragma unroll
     for (int e = 0; e < VN; ++e) count(IDENT ? Vec16<U>::get(v, e) : to_ordered(Vec16<U>::get(v, e), xf));
@@ -110,7 +119,7 @@ __global__ __launch_bounds__(kHistThreads) void radix_hist_kernel(const U* __res
   __syncthreads();
   // One thread per digit pair: the 32 copies summed, read in an order
   // rotated by thread so that a wave's reads spread over the banks.
-  for (uint32_t w = tid; w < (uint32_t)passes * (kRadix / 2); w += kHistThreads) {
+  for (uint32_t w = tid; w < (uint32_t)(MAXP - LOW) * (kRadix / 2); w += kHistThreads) {
     uint32_t lo = 0, hi = 0;
 #pragma unroll 8
     for (uint32_t c = 0; c < 32; ++c) {
@@ -118,10 +127,30 @@ __global__ __launch_bounds__(kHistThreads) void radix_hist_kernel(const U* __res
       lo += x & 0xFFFFu;
       hi += x >> 16;
     }
-    const uint32_t p = w / (kRadix / 2), d = (w % (kRadix / 2)) * 2;
+    const uint32_t p = LOW + w / (kRadix / 2), d = (w % (kRadix / 2)) * 2;
     if (lo) atomicAdd(&g_hist[p * kRadix + d], (unsigned long long)lo);
     if (hi) atomicAdd(&g_hist[p * kRadix + d + 1], (unsigned long long)hi);
   }
+}
+
+template <bool IDENT>
+__global__ __launch_bounds__(kHistThreads) void radix_hist_kernel(const uint64_t* __restrict__ keys, uint64_t n,
+                                                                  Xform<uint64_t> xf, const SortCtrl* ctrl,
+                                                                  unsigned long long* __restrict__ g_hist,
+                                                                  uint4* __restrict__ zero_ptr, uint64_t zero_vec4) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_cnt[8 * (kRadix / 2) * 32];
+  const uint32_t low = ctrl->low();
+  const uint64_t gtid = (uint64_t)blockIdx.x * kHistThreads + threadIdx.x;
+  const uint64_t gstride = (uint64_t)gridDim.x * kHistThreads;
+  for (uint64_t i = gtid; i < zero_vec4; i += gstride) zero_ptr[i] = make_uint4(0, 0, 0, 0);
+  if (low >= 6)
+    radix_hist_from<IDENT, 6>(keys, n, xf, g_hist, s_cnt);
+  else if (low >= 4)
+    radix_hist_from<IDENT, 4>(keys, n, xf, g_hist, s_cnt);
+  else if (low >= 2)
+    radix_hist_from<IDENT, 2>(keys, n, xf, g_hist, s_cnt);
+  else
+    radix_hist_from<IDENT, 0>(keys, n, xf, g_hist, s_cnt);
 }
 
 // 32-bit keys: full 32-bit counters (no packing, so an add is a constant 1
@@ -181,50 +210,90 @@ __global__ __launch_bounds__(kHistThreads) void radix_hist32_kernel(const uint32
 }
 
 // Workgroups of the histogram kernel: at most kHistKeysPerThread keys per
-// thread (the 16-bit count bound), and up to 512 workgroups to spread the
-// read over the chip.
+// thread (the 16-bit count bound), at least 8 where there are not 512
+// workgroups of them: each ends with an atomic add per counter, which at 2^20
+// 64-bit keys on 512 workgroups was most of its 31 us (on 123: 12.7; 10^6
+// 32-bit keys 9.4 -> 6).
+constexpr uint64_t kHistKeysMin = 8;
 static uint64_t hist_blocks_for(uint64_t n) {
   const uint64_t per_block = (uint64_t)kHistThreads * kHistKeysPerThread;
   uint64_t blocks = (n + per_block - 1) / per_block;
-  const uint64_t spread = (n + kHistThreads - 1) / kHistThreads;
+  const uint64_t spread = (n + kHistThreads * kHistKeysMin - 1) / (kHistThreads * kHistKeysMin);
   const uint64_t floor = spread < 512 ? spread : 512;
   if (blocks < floor) blocks = floor;
   return blocks < 1 ? 1 : blocks;
 }
 
-__global__ __launch_bounds__(256) void radix_scan_kernel(const unsigned long long* __restrict__ g_hist,
-                                                         uint64_t* __restrict__ digit_base, SortCtrl* ctrl,
-                                                         int passes, uint64_t n) {
-  __shared__ uint64_t s_wsum[4];
-  __shared__ uint32_t s_trivial[kMaxPasses];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int p = 0; p < passes; ++p) {
-    const uint64_t c = g_hist[p * kRadix + tid];
-    const uint64_t incl = wave_incl_scan64(c);
-    if (lane == 63) s_wsum[wave] = incl;
-    __syncthreads();
-    uint64_t add = 0;
-    for (uint32_t w = 0; w < wave; ++w) add += s_wsum[w];
-    digit_base[p * kRadix + tid] = incl - c + add;
-    const int trivial = __syncthreads_or(c == n);
-    if (tid == 0) s_trivial[p] = trivial;
-    __syncthreads();
+// Exclusive starts of the 256 digits of one digit position by one wave, four
+// digits a lane; true if one digit holds all n keys.
+__device__ inline bool scan_digits(const unsigned long long* __restrict__ hist, uint64_t* __restrict__ base,
+                                   uint64_t n) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const ulonglong2 a = reinterpret_cast<const ulonglong2*>(hist)[2 * lane];
+  const ulonglong2 b = reinterpret_cast<const ulonglong2*>(hist)[2 * lane + 1];
+  const uint64_t sum = a.x + a.y + b.x + b.y;
+  uint64_t run = wave_incl_scan64(sum) - sum;
+  base[4 * lane] = run;
+  base[4 * lane + 1] = run += a.x;
+  base[4 * lane + 2] = run += a.y;
+  base[4 * lane + 3] = run += b.x;
+  return ballot(a.x == n || a.y == n || b.x == n || b.y == n) != 0;
+}
+
+// First launch of a sort: zeroes the digit histograms and, with `keys` (64-bit
+// keys, block 0), picks the lowest digit to sort by.
+__global__ __launch_bounds__(256) void radix_prep_kernel(uint32_t* __restrict__ g_hist, uint32_t words, SortCtrl* ctrl,
+                                                         const uint64_t* __restrict__ keys, uint64_t n,
+                                                         Xform<uint64_t> xf) {
+  __shared__ LowTile::Smem s_tile;
+  __shared__ uint32_t s_sum[8];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = blockIdx.x * 256 + tid; i < words; i += gridDim.x * 256) g_hist[i] = 0;
+  if (blockIdx.x != 0) return;
+  uint32_t low = 0;
+  if (keys) {
+    uint64_t k[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      k[i] = to_ordered(keys[sample_pos((tid >> 6) * 256 + (uint32_t)i * 64 + (tid & 63u), n)], xf);
+    low = choose_low(s_tile, k, n, false, s_sum);
   }
   if (tid == 0) {
-    uint32_t sel = 0, run = 0;
-    for (int p = 0; p < kMaxPasses; ++p) {
-      ctrl->tile_counter[p] = 0;
-      for (int c = 0; c < 8; ++c) ctrl->class_counter[p][c] = 0;
-      if (p >= passes || s_trivial[p]) {
-        ctrl->src[p] = kSkipPass;
-      } else {
-        ctrl->src[p] = sel;
-        sel ^= 1u;
-        ++run;
-      }
+    ctrl->top_digits = low ? 8 - low : 0;
+    ctrl->long_count = 0;
+  }
+}
+
+// Digit starts of every pass (a wave per digit position), and which passes
+// run: not those whose digit is the same for every key, nor those below the
+// lowest digit sorted by.
+__global__ __launch_bounds__(256) void radix_scan_kernel(const unsigned long long* __restrict__ g_hist,
+                                                         uint64_t* __restrict__ digit_base, SortCtrl* ctrl, int passes,
+                                                         uint64_t n) {
+  __shared__ uint32_t s_trivial[kMaxPasses];
+  const uint32_t tid = threadIdx.x, wave = tid >> 6;
+  const uint32_t low = ctrl->low();
+  if (tid < kMaxPasses) s_trivial[tid] = 1;
+  if (tid < kMaxPasses * 8) ctrl->class_counter[tid / 8][tid % 8] = 0;
+  __syncthreads();
+  for (int p = (int)wave; p < passes; p += 4) {
+    const bool trivial = scan_digits(g_hist + p * kRadix, digit_base + p * kRadix, n);
+    if ((tid & 63u) == 0) s_trivial[p] = trivial || (uint32_t)p < low;
+  }
+  __syncthreads();
+  if (tid < kMaxPasses) {
+    uint32_t before = 0, run = 0;  // passes that run before this one, and in all
+    for (uint32_t p = 0; p < kMaxPasses; ++p) {
+      const uint32_t r = s_trivial[p] ? 0u : 1u;
+      before += p < tid ? r : 0u;
+      run += r;
     }
-    ctrl->final_sel = sel;
-    ctrl->passes_run = run;
+    ctrl->tile_counter[tid] = 0;
+    ctrl->src[tid] = s_trivial[tid] ? kSkipPass : (before & 1u);
+    if (tid == 0) {
+      ctrl->final_sel = run & 1u;
+      ctrl->passes_run = run;
+    }
   }
 }
 
@@ -487,6 +556,9 @@ __global__ __launch_bounds__(THREADS) void onesweep_kernel(OnesweepArgs<U, V, S>
   }
 
   uint32_t src;
+  if constexpr (SEG && sizeof(U) == 8) {
+    if ((uint32_t)a.pass < a.ctrl->low()) return;  // a digit below the lowest one sorted by (radix_ties.h)
+  }
   if constexpr (SPLIT) {
     src = 0;
   } else if constexpr (SEG) {
@@ -1071,8 +1143,13 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
   S* status = reinterpret_cast<S*>(ws + L.off_status);
   const uint64_t status_per_pass = L.tiles * kRadix;
 
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(8), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
-                     (uint64_t)(kMaxPasses * kRadix * 2), 0u);
+  if constexpr (sizeof(U) == 8)
+    hipLaunchKernelGGL(radix_prep_kernel, dim3(8), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
+                       (uint32_t)(kMaxPasses * kRadix * 2), ctrl, n >= 4 * kLowSample ? (const U*)keys : nullptr, n, xf);
+  else
+    hipLaunchKernelGGL(radix_prep_kernel, dim3(8), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
+                       (uint32_t)(kMaxPasses * kRadix * 2), ctrl, (const uint64_t*)nullptr, n,
+                       Xform<uint64_t>{0, 0, 0});
   const uint64_t status_bytes = (uint64_t)L.passes * status_per_pass * sizeof(S);
   const uint64_t hist_blocks = hist_blocks_for(n);
   // The histogram kernel counts every key byte (L.passes == sizeof(U)).
@@ -1089,11 +1166,11 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
                          reinterpret_cast<const uint32_t*>(keys), n, *reinterpret_cast<const Xform<uint32_t>*>(&xf),
                          hist, reinterpret_cast<uint4*>(status), status_bytes / 16);
   } else if (ident)
-    hipLaunchKernelGGL((radix_hist_kernel<U, true>), dim3((uint32_t)hist_blocks), dim3(kHistThreads), 0, stream, keys,
-                       n, xf, L.passes, hist, reinterpret_cast<uint4*>(status), status_bytes / 16);
+    hipLaunchKernelGGL((radix_hist_kernel<true>), dim3((uint32_t)hist_blocks), dim3(kHistThreads), 0, stream, keys, n,
+                       xf, ctrl, hist, reinterpret_cast<uint4*>(status), status_bytes / 16);
   else
-    hipLaunchKernelGGL((radix_hist_kernel<U, false>), dim3((uint32_t)hist_blocks), dim3(kHistThreads), 0, stream,
-                       keys, n, xf, L.passes, hist, reinterpret_cast<uint4*>(status), status_bytes / 16);
+    hipLaunchKernelGGL((radix_hist_kernel<false>), dim3((uint32_t)hist_blocks), dim3(kHistThreads), 0, stream, keys, n,
+                       xf, ctrl, hist, reinterpret_cast<uint4*>(status), status_bytes / 16);
   if (timer) timer->end(stream);
   hipLaunchKernelGGL(radix_scan_kernel, dim3(1), dim3(256), 0, stream, hist, base, ctrl, L.passes, n);
   for (int p = 0; p < L.passes; ++p) {
@@ -1120,8 +1197,22 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
                          dim3(THREADS), 0, stream, a);
     if (timer) timer->end(stream);
   }
+  if constexpr (sizeof(U) == 8) {
+    TieArgs<V> t{};
+    t.keys0 = keys;
+    t.keys1 = keys_tmp;
+    t.vals0 = vals;
+    t.vals1 = vals_tmp;
+    t.n = n;
+    t.xf = xf;
+    t.ctrl = ctrl;
+    t.use_status(status, status_per_pass * sizeof(S), L.tiles, THREADS * ITEMS);
+    // One chunk a workgroup up to 2^23 keys (four a CU at 2^21), then four.
+    t.tile_keys = n <= (1ull << 23) ? kTieChunk : 4 * kTieChunk;
+    launch_tie_fix<V, KV>(t, (n + t.tile_keys - 1) / t.tile_keys, n, stream, timer);
+  }
   uint64_t copy_blocks = (n + 255) / 256;
-  if (copy_blocks > 4096) copy_blocks = 4096;
+  if (copy_blocks > 1024) copy_blocks = 1024;  // reads one word and leaves where no copy is due
   hipLaunchKernelGGL((radix_final_copy_kernel<U, V, KV>), dim3((uint32_t)copy_blocks), dim3(256), 0, stream, keys,
                      keys_tmp, vals, vals_tmp, n, ctrl);
   return hipGetLastError();
@@ -1181,6 +1272,7 @@ struct SegHistArgs {
   uint32_t* seg_cnt;  // [slot][pass][256]
   uint32_t* status;   // [pass][tile][256]
   uint64_t status_per_pass;
+  const SortCtrl* ctrl;
 };
 
 // Digit counts of one tile for every pass, added into its segment's counts
@@ -1192,15 +1284,12 @@ struct SegHistArgs {
 // (runs of equal keys) is added once per digit by one lane.
 constexpr uint32_t kSegHistCopies = 4;
 
-template <typename U, bool IDENT>
-__global__ __launch_bounds__(256) void seg_hist_kernel(SegHistArgs<U> a) {
-  constexpr int MAXP = sizeof(U);  // one 8-bit digit per key byte (passes == MAXP)
-  __shared__ uint32_t s_hist[MAXP * kRadix * kSegHistCopies];  // [pass][digit][copy]
+template <typename U, bool IDENT, int LOW>
+__device__ __forceinline__ void seg_hist_from(const SegHistArgs<U>& a, uint32_t* s_hist) {  // [digit][value][copy]
+  constexpr int MAXP = sizeof(U);  // one 8-bit digit per key byte (passes == MAXP); those from LOW up are counted
   const uint32_t tid = threadIdx.x, tile = blockIdx.x;
   const uint32_t copy = tid & (kSegHistCopies - 1);
-  const int passes = a.passes;
-  for (uint32_t i = tid; i < (uint32_t)MAXP * kRadix * kSegHistCopies; i += 256) s_hist[i] = 0;
-  for (int p = 0; p < passes; ++p) a.status[p * a.status_per_pass + (uint64_t)tile * kRadix + tid] = 0;
+  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * kRadix * kSegHistCopies; i += 256) s_hist[i] = 0;
   const uint32_t slot = a.tile_seg[tile];
   const uint64_t start = a.seg_range[2 * slot] + (uint64_t)(tile - a.seg_first[slot]) * a.tile_keys;
   const uint64_t seg_end = a.seg_range[2 * slot + 1];
@@ -1217,12 +1306,13 @@ __global__ __launch_bounds__(256) void seg_hist_kernel(SegHistArgs<U> a) {
     if (ballot(u == u0) == active) {
       if (count_below(active) == 0) {
 #pragma unroll
-        for (int p = 0; p < MAXP; ++p)
-          atomicAdd(&s_hist[(p * kRadix + digit_of(u, p * 8)) * kSegHistCopies], (uint32_t)__popcll(active));
+        for (int p = LOW; p < MAXP; ++p)
+          atomicAdd(&s_hist[((p - LOW) * kRadix + digit_of(u, p * 8)) * kSegHistCopies], (uint32_t)__popcll(active));
       }
     } else {
 #pragma unroll
-      for (int p = 0; p < MAXP; ++p) atomicAdd(&s_hist[(p * kRadix + digit_of(u, p * 8)) * kSegHistCopies + copy], 1u);
+      for (int p = LOW; p < MAXP; ++p)
+        atomicAdd(&s_hist[((p - LOW) * kRadix + digit_of(u, p * 8)) * kSegHistCopies + copy], 1u);
     }
   };
   // Four keys per thread in flight: the loads are issued before any is
@@ -1237,8 +1327,8 @@ __global__ __launch_bounds__(256) void seg_hist_kernel(SegHistArgs<U> a) {
   }
   for (; i < end; i += 256) count(a.keys[i]);
   __syncthreads();
-  uint32_t* dst = a.seg_cnt + (uint64_t)slot * passes * kRadix;
-  for (uint32_t i = tid; i < (uint32_t)passes * kRadix; i += 256) {
+  uint32_t* dst = a.seg_cnt + (uint64_t)slot * a.passes * kRadix + LOW * kRadix;
+  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * kRadix; i += 256) {
     uint32_t c = 0;
 #pragma unroll
     for (uint32_t j = 0; j < kSegHistCopies; ++j) c += s_hist[i * kSegHistCopies + j];
@@ -1250,21 +1340,56 @@ __global__ __launch_bounds__(256) void seg_hist_kernel(SegHistArgs<U> a) {
   }
 }
 
+template <typename U, bool IDENT>
+__global__ __launch_bounds__(256) void seg_hist_kernel(SegHistArgs<U> a) {
+  __shared__ uint32_t s_hist[sizeof(U) * kRadix * kSegHistCopies];
+  const uint32_t tid = threadIdx.x, tile = blockIdx.x;
+  for (int p = 0; p < a.passes; ++p) a.status[p * a.status_per_pass + (uint64_t)tile * kRadix + tid] = 0;
+  if constexpr (sizeof(U) == 8) {
+    const uint32_t low = a.ctrl->low();
+    if (low >= 4) return seg_hist_from<U, IDENT, 4>(a, s_hist);
+    if (low >= 2) return seg_hist_from<U, IDENT, 2>(a, s_hist);
+  }
+  seg_hist_from<U, IDENT, 0>(a, s_hist);
+}
+
+// The lowest digit to sort by of the first kLowSlots multi-tile segments of
+// 64-bit keys, a workgroup each (four or six digits, so that the result lands
+// where the keys were): the largest number of digits counts.
+constexpr uint32_t kLowSlots = 2048;
+
+__global__ __launch_bounds__(256) void seg_prep_kernel(SortCtrl* ctrl, const uint64_t* __restrict__ keys,
+                                                       const uint64_t* __restrict__ seg_range, Xform<uint64_t> xf) {
+  __shared__ LowTile::Smem s_tile;
+  __shared__ uint32_t s_sum[8];
+  const uint32_t tid = threadIdx.x;
+  const uint64_t start = seg_range[2 * blockIdx.x];
+  const uint64_t len = seg_range[2 * blockIdx.x + 1] - start;
+  uint64_t k[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    k[i] = to_ordered(keys[start + sample_pos((tid >> 6) * 256 + (uint32_t)i * 64 + (tid & 63u), len)], xf);
+  uint32_t low = choose_low(s_tile, k, len, true, s_sum);
+  low = low > 4 ? 4 : low;
+  if (tid == 0) atomicMax(&ctrl->top_digits, 8 - low);
+}
+
 // Counts -> exclusive digit starts within the segment, in place, one
-// workgroup per segment; block 0 also resets the pass tickets.
+// workgroup per segment and a wave per digit position; block 0 also resets
+// the pass tickets.
 __global__ __launch_bounds__(256) void seg_scan_kernel(uint32_t* seg_cnt, int passes, SortCtrl* ctrl) {
-  __shared__ uint32_t s_wsum[4];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   uint32_t* c = seg_cnt + (uint64_t)blockIdx.x * passes * kRadix;
-  for (int p = 0; p < passes; ++p) {
-    const uint32_t x = c[p * kRadix + tid];
-    const uint32_t incl = wave_incl_scan(x);
-    if (lane == 63) s_wsum[wave] = incl;
-    __syncthreads();
-    uint32_t add = 0;
-    for (uint32_t w = 0; w < wave; ++w) add += s_wsum[w];
-    c[p * kRadix + tid] = incl - x + add;
-    __syncthreads();
+  for (int p = (int)wave; p < passes; p += 4) {
+    uint4* const row = reinterpret_cast<uint4*>(c + p * kRadix) + lane;
+    const uint4 x = *row;
+    const uint32_t sum = x.x + x.y + x.z + x.w;
+    uint4 y;
+    y.x = wave_incl_scan_dpp(sum) - sum;
+    y.y = y.x + x.x;
+    y.z = y.y + x.y;
+    y.w = y.z + x.z;
+    *row = y;
   }
   if (blockIdx.x == 0 && tid < kMaxPasses) ctrl->tile_counter[tid] = 0;
   if (blockIdx.x == 0 && tid < kMaxPasses * 8) ctrl->class_counter[tid / 8][tid % 8] = 0;
@@ -1316,9 +1441,15 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
   // geometry's tile, or the tile maps and status words would not fit it.
   if (radix_seg_tile_keys((int)sizeof(U), VB, G) != (uint32_t)(THREADS * ITEMS)) return hipErrorInvalidValue;
 
-  if (T.n_multi) {
-    hipError_t e = fill_u32(cnt, (uint64_t)T.n_multi * L.passes * kRadix, 0u, stream);
-    if (e != hipSuccess) return e;
+  // Clears the control block and the multi-tile counts.
+  hipError_t e = fill_u32(reinterpret_cast<uint32_t*>(ws + L.off_ctrl),
+                          (L.off_cnt - L.off_ctrl) / 4 + (uint64_t)T.n_multi * L.passes * kRadix, 0u, stream);
+  if (e != hipSuccess) return e;
+  // Every multi-tile segment holds more than a sample's keys.
+  const uint32_t sampled = sizeof(U) == 8 ? std::min(T.n_multi, kLowSlots) : 0;
+  if constexpr (sizeof(U) == 8) {
+    if (sampled)
+      hipLaunchKernelGGL(seg_prep_kernel, dim3(sampled), dim3(256), 0, stream, ctrl, (const U*)keys, T.seg_range, xf);
   }
   SegHistArgs<U> h;
   h.keys = keys;
@@ -1332,6 +1463,7 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
   h.seg_cnt = cnt;
   h.status = status;
   h.status_per_pass = status_per_pass;
+  h.ctrl = ctrl;
   if (timer) timer->begin("seg_hist", T.n_keys * sizeof(U), stream);
   if (ident)
     hipLaunchKernelGGL((seg_hist_kernel<U, true>), dim3((uint32_t)T.tiles), dim3(256), 0, stream, h);
@@ -1367,6 +1499,23 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
       hipLaunchKernelGGL((onesweep_kernel<U, V, KV, THREADS, ITEMS, uint32_t, false, true, Idx>),
                          dim3((uint32_t)T.tiles), dim3(THREADS), 0, stream, a);
     if (timer) timer->end(stream);
+  }
+  if constexpr (sizeof(U) == 8) {
+    if (sampled) {
+      TieArgs<V> t{};
+      t.keys0 = keys;
+      t.keys1 = reinterpret_cast<U*>(ws + L.off_keys_tmp);
+      t.vals0 = reinterpret_cast<V*>(vals_v);
+      t.vals1 = reinterpret_cast<V*>(ws + L.off_vals_tmp);
+      t.xf = xf;
+      t.ctrl = ctrl;
+      t.tile_keys = THREADS * ITEMS;
+      t.tile_seg = T.tile_seg;
+      t.seg_first = T.seg_first;
+      t.seg_range = T.seg_range;
+      t.use_status(status, status_per_pass * sizeof(uint32_t), T.tiles, THREADS * ITEMS);
+      launch_tie_fix<V, KV>(t, T.tiles, T.n_keys, stream, timer);
+    }
   }
   return hipGetLastError();
 }
@@ -1562,8 +1711,8 @@ static hipError_t multisplit_t(const U* keys, const void* vals, uint64_t n, cons
   unsigned long long* hist = reinterpret_cast<unsigned long long*>(ws + L.off_hist);
   uint64_t* base = d_bucket_base ? d_bucket_base : reinterpret_cast<uint64_t*>(ws + L.off_base);
   S* status = reinterpret_cast<S*>(ws + L.off_status);
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
-                     (uint64_t)(kRadix * 2), 0u);
+  hipLaunchKernelGGL(radix_prep_kernel, dim3(1), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
+                     (uint32_t)(kRadix * 2), ctrl, (const uint64_t*)nullptr, n, Xform<uint64_t>{0, 0, 0});
   const uint64_t status_bytes = L.tiles * kRadix * sizeof(S);
   uint64_t blocks = (n + kSplitHistThreads * 16 - 1) / (kSplitHistThreads * 16);
   if (blocks < 1) blocks = 1;
