@@ -156,6 +156,39 @@ gs_status sort_device(gs_handle* h, gs_dtype kdt, void* d_keys, gs_dtype vdt, vo
                   "radix sort");
 }
 
+// The direct gather takes no scratch, so it stands in wherever the scratch
+// cannot be had: under stream capture (the graph would keep a pointer to a
+// block that a later call may replace) and out of memory.
+hipError_t gather_device(gs_handle* h, int elem_bytes, const void* src, const uint64_t* idx, void* dst, uint64_t n) {
+  const size_t bytes = gather_split_bytes(elem_bytes, n);
+  if (bytes == 0) return gather_values(elem_bytes, src, idx, dst, n, h->stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+  if (hipStreamIsCapturing(h->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return gather_values(elem_bytes, src, idx, dst, n, h->stream);
+  }
+  std::lock_guard<std::mutex> lock(h->gather_mutex);
+  // Allocating must not end a capture under way on another thread.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  void* ws = nullptr;
+  hipError_t e = hipSuccess;
+  if (h->gather_done == nullptr)
+    e = hipEventCreateWithFlags(&h->gather_done, hipEventDisableTiming);
+  else if (h->stream != h->gather_stream)
+    e = hipStreamWaitEvent(h->stream, h->gather_done, 0);
+  if (e == hipSuccess) e = h->arena.get(Arena::kGather, bytes, h->stream, &ws);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return gather_values(elem_bytes, src, idx, dst, n, h->stream);
+  }
+  e = gather_split(elem_bytes, src, idx, dst, n, ws, h->stream);
+  h->gather_stream = h->stream;
+  const hipError_t rec = hipEventRecord(h->gather_done, h->stream);
+  return e != hipSuccess ? e : rec;
+}
+
 // ------------------------------------------------------------ host chunks
 //
 // Host-memory sorts of inputs larger than the device can stage, as the
@@ -408,6 +441,7 @@ gs_status gs_destroy(gs_handle* h) {
     (void)hipStreamSynchronize(h->stream);
     h->arena.release();
     if (h->pinned) (void)hipHostFree(h->pinned);
+    if (h->gather_done) (void)hipEventDestroy(h->gather_done);
   }
   delete h;
   return GS_OK;
@@ -692,7 +726,7 @@ gs_status gs_gather(gs_handle* h, int elem_bytes, const void* d_src, const uint6
   DeviceScope ds(h->device);
   LaunchTimer* t = h->timer();
   if (t) t->begin("gather", n * (8 + 2 * (uint64_t)elem_bytes), h->stream);
-  const hipError_t e = gather_values(elem_bytes, d_src, d_idx, d_dst, n, h->stream);
+  const hipError_t e = gather_device(h, elem_bytes, d_src, d_idx, d_dst, n);
   if (t) t->end(h->stream);
   return from_hip(e, "gather");
 }

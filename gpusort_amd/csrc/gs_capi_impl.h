@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -42,7 +43,7 @@ class Profiler : public LaunchTimer {
 class Arena {
  public:
   enum Slot { kRadix = 0, kStageKeys, kStageVals, kStagePairs, kMerge, kSmall, kPipeKeys, kPipeVals, kPipeAux,
-              kSegAux, kSegWork, kHykWork, kSlots };
+              kSegAux, kSegWork, kHykWork, kGather, kSlots };
   Arena() {
     for (int i = 0; i < kSlots; ++i) {
       ptr_[i] = nullptr;
@@ -85,6 +86,9 @@ int val_bytes_of(gs_dtype d);
 hipError_t noalloc_setup(int device);
 gs_status sort_device(gs_handle* h, gs_dtype kdt, void* d_keys, gs_dtype vdt, void* d_vals, uint64_t n,
                       int descending);
+// dst[i] = src[idx[i]] queued on h->stream, through source regions where that
+// pays and its scratch can be had.
+hipError_t gather_device(gs_handle* h, int elem_bytes, const void* src, const uint64_t* idx, void* dst, uint64_t n);
 // Segmented sort from host offsets, queued on h->stream without waiting;
 // `meta` must outlive the queued work; segments of 2^30+ keys are returned
 // in `huge` for the caller to sort.
@@ -104,6 +108,11 @@ struct gs_handle {
   // 0: the device's free memory at the call.
   uint64_t host_budget = 0;
   gs::Arena arena;
+  // The gather's scratch: gathers from several threads queue one after
+  // another, and one on another stream than the last waits for it.
+  std::mutex gather_mutex;
+  hipEvent_t gather_done = nullptr;
+  hipStream_t gather_stream = nullptr;
   gs::Profiler profiler;
   gs::LaunchTimer* timer() { return profiler.active ? &profiler : nullptr; }
   void* pinned = nullptr;

@@ -306,6 +306,12 @@ hipError_t fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t stream);
 hipError_t copy_bytes(void* dst, const void* src, uint64_t bytes, hipStream_t stream);
 hipError_t gather_values(int val_bytes, const void* src, const uint64_t* idx, void* dst, uint64_t n,
                          hipStream_t stream);
+// The same for large n through source regions (gather.hip): bytes of scratch,
+// 0 where gather_values is the faster one, and the gather.
+constexpr uint64_t kGatherSplitMin = 1ull << 24;
+size_t gather_split_bytes(int elem_bytes, uint64_t n);
+hipError_t gather_split(int elem_bytes, const void* src, const uint64_t* idx, void* dst, uint64_t n, void* workspace,
+                        hipStream_t stream);
 hipError_t pack_pairs(int key_bytes, const void* keys, int val_bytes, const void* vals, void* out, uint64_t n,
                       uint32_t stride_bytes, uint32_t val_offset, hipStream_t stream);
 hipError_t iota_u64(uint64_t* out, uint64_t n, uint64_t base, hipStream_t stream);

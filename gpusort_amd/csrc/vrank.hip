@@ -904,7 +904,7 @@ extern "C" gs_status gs_gather_host(gs_handle* h, int elem_bytes, const void* h_
   hipError_t e = hipMemcpyAsync(ds_src, h_src, n_src * (size_t)elem_bytes, hipMemcpyHostToDevice, h->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(ds_idx, h_idx, n * 8, hipMemcpyHostToDevice, h->stream);
   if (e == hipSuccess)
-    e = gather_values(elem_bytes, ds_src, reinterpret_cast<const uint64_t*>(ds_idx), ds_dst, n, h->stream);
+    e = gather_device(h, elem_bytes, ds_src, reinterpret_cast<const uint64_t*>(ds_idx), ds_dst, n);
   if (e == hipSuccess) e = hipMemcpyAsync(h_dst, ds_dst, n * (size_t)elem_bytes, hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   return from_hip(e, "gather");

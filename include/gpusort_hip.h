@@ -316,7 +316,9 @@ gs_status gs_vrank_sort_host(gs_handle* h, gs_algorithm algo, gs_dtype kdt, void
                              int descending, gs_vrank_report* report);
 
 /* dst[i] = src[idx[i]] for a payload of elem_bytes (1, 2, 4, 8) bytes.
- * Device form of ParUtils::ArrangeValues (include/par/par_utils.h:22-86). */
+ * Device form of ParUtils::ArrangeValues (include/par/par_utils.h:22-86).
+ * From 2^24 elements it takes 6 bytes an element of the handle's arena (none
+ * under stream capture or where they cannot be had: it is slower then). */
 gs_status gs_gather(gs_handle* h, int elem_bytes, const void* d_src, const uint64_t* d_idx, void* d_dst,
                     uint64_t n);
 
