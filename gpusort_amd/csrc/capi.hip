@@ -624,26 +624,11 @@ gs_status gs_merge(gs_handle* h, gs_dtype kdt, const void* a_k, const void* a_v,
   DeviceScope ds(h->device);
   const int kb = dtype_bytes(kdt), vb = val_bytes_of(vdt);
   const XformParams xf = make_xform((int)kdt, descending != 0);
-  MergeJob job{0, na, 0, nb, 0};
-  MergeJobDev dj[1];
-  std::vector<uint32_t> tile_job;
-  const uint32_t ntiles = merge_plan(&job, 1, dj, &tile_job);
-  const size_t bytes = align_up(sizeof(MergeJobDev), 256) + align_up(ntiles * sizeof(uint32_t), 256) +
-                       align_up((size_t)ntiles * sizeof(uint64_t), 256);
   void* ws = nullptr;
-  hipError_t e = h->arena.get(Arena::kMerge, bytes, h->stream, &ws);
+  hipError_t e = h->arena.get(Arena::kMerge, merge_two_tiles(kb, vb, total) * sizeof(uint64_t), h->stream, &ws);
   if (e != hipSuccess) return from_hip(e, "merge workspace");
-  char* w = reinterpret_cast<char*>(ws);
-  MergeJobDev* d_jobs = reinterpret_cast<MergeJobDev*>(w);
-  uint32_t* d_tile_job = reinterpret_cast<uint32_t*>(w + align_up(sizeof(MergeJobDev), 256));
-  uint64_t* d_split = reinterpret_cast<uint64_t*>(w + align_up(sizeof(MergeJobDev), 256) +
-                                                  align_up(ntiles * sizeof(uint32_t), 256));
-  e = hipMemcpyAsync(d_jobs, dj, sizeof(MergeJobDev), hipMemcpyHostToDevice, h->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(d_tile_job, tile_job.data(), ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, h->stream);
-  if (e == hipSuccess)
-    e = merge_tiles(kb, vb, a_k, b_k, a_v, b_v, o_k, o_v, d_jobs, d_tile_job, ntiles, xf, d_split, h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);  // the host job table is stack memory
+  e = merge_two(kb, vb, a_k, a_v, na, b_k, b_v, nb, o_k, o_v, xf, reinterpret_cast<uint64_t*>(ws), h->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   return from_hip(e, "merge");
 }
 

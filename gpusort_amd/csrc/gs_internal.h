@@ -163,9 +163,10 @@ struct MergeJobDev {
 };
 
 // Output elements per merge tile.
-uint32_t merge_tile_elems();
+uint32_t merge_tile_elems(int key_bytes, int val_bytes);
 // Fills out_jobs[0..njobs) and the tile -> job table; returns the tile count.
-uint32_t merge_plan(const MergeJob* jobs, uint32_t njobs, MergeJobDev* out_jobs, std::vector<uint32_t>* tile_job);
+uint32_t merge_plan(int key_bytes, int val_bytes, const MergeJob* jobs, uint32_t njobs, MergeJobDev* out_jobs,
+                    std::vector<uint32_t>* tile_job);
 // Runs every job: run a of a job is read from keys_a/vals_a + a_off, run b
 // from keys_b/vals_b + b_off.  d_split needs ntiles entries of scratch.
 // lex_vxf: when given (and there is a payload) elements compare as (key,
@@ -174,6 +175,13 @@ hipError_t merge_tiles(int key_bytes, int val_bytes, const void* keys_a, const v
                        const void* vals_b, void* dst_keys, void* dst_vals, const MergeJobDev* d_jobs,
                        const uint32_t* d_tile_job, uint32_t ntiles, const XformParams& xf, uint64_t* d_split,
                        hipStream_t stream, const XformParams* lex_vxf = nullptr);
+
+// One job of n elements in all, with nothing to upload: d_split needs
+// merge_two_tiles() entries.
+uint64_t merge_two_tiles(int key_bytes, int val_bytes, uint64_t n);
+hipError_t merge_two(int key_bytes, int val_bytes, const void* keys_a, const void* vals_a, uint64_t na,
+                     const void* keys_b, const void* vals_b, uint64_t nb, void* dst_keys, void* dst_vals,
+                     const XformParams& xf, uint64_t* d_split, hipStream_t stream);
 
 // One merge-split of SampleSort's small-input bitonic network: rank list a
 // (own) and b (partner), both sorted, in one device buffer.

@@ -45,36 +45,77 @@ struct MKey {
   }
 };
 
+// Where a merge's jobs are: a list with a tile -> job table, or, for one job,
+// the job itself among the kernel's arguments (no table, nothing to upload).
+struct MergeJobs {
+  const MergeJobDev* list;  // null: one
+  const uint32_t* tile_job;
+  MergeJobDev one;
+  __device__ MergeJobDev of(uint32_t tile) const { return list ? list[tile_job[tile]] : one; }
+};
+
+// The split of every tile's first diagonal: kSplitLanes lanes search together,
+// each probing one of kSplitLanes evenly spaced places a round.  What bounds it
+// is the chain of dependent reads: 7 rounds for 2^25 elements where one lane
+// alone takes 26, which were 31 us of a merge of 2^25 + 2^24 pairs.
+constexpr uint32_t kSplitLanes = 16;
+
 template <typename U, typename V, bool LEX>
 __global__ __launch_bounds__(256) void merge_partition_kernel(const U* __restrict__ keys_a,
                                                               const U* __restrict__ keys_b,
                                                               const V* __restrict__ vals_a,
-                                                              const V* __restrict__ vals_b,
-                                                              const MergeJobDev* __restrict__ jobs,
-                                                              const uint32_t* __restrict__ tile_job,
+                                                              const V* __restrict__ vals_b, MergeJobs jobs,
                                                               uint32_t ntiles, uint32_t tile_elems, Xform<U> xf,
                                                               Xform<V> vxf, uint64_t* __restrict__ a_split) {
-  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= ntiles) return;
-  const MergeJobDev jb = jobs[tile_job[t]];
-  const uint64_t diag = (uint64_t)(t - jb.tile0) * tile_elems;
+  const uint32_t t = (blockIdx.x * 256 + threadIdx.x) / kSplitLanes;
+  const uint32_t lane = threadIdx.x % kSplitLanes;
+  const uint32_t shift = lane_id() / kSplitLanes * kSplitLanes;
+  const bool in = t < ntiles;  // the lanes of a wave stay together
+  const MergeJobDev jb = jobs.of(in ? t : ntiles - 1);
+  const uint64_t diag = in ? (uint64_t)(t - jb.tile0) * tile_elems : 0;
   const U* A = keys_a + jb.a_off;
   const U* B = keys_b + jb.b_off;
   const V* AV = vals_a + jb.a_off;
   const V* BV = vals_b + jb.b_off;
   using E = MKey<U, V, LEX>;
-  a_split[t] = merge_path_search<E>(
-      diag, jb.a_len, jb.b_len,
-      [&](uint64_t i) { return E{to_ordered(A[i], xf), LEX ? to_ordered(AV[i], vxf) : V(0)}; },
-      [&](uint64_t i) { return E{to_ordered(B[i], xf), LEX ? to_ordered(BV[i], vxf) : V(0)}; });
+  // The first place in [lo, hi] where A's element comes after B's (hi if none).
+  uint64_t lo = diag > jb.b_len ? diag - jb.b_len : 0;
+  uint64_t hi = diag < jb.a_len ? diag : jb.a_len;
+  while (ballot(lo < hi)) {
+    // Places lo + (hi - lo) * (lane + 1) / 17, in order, below hi while lo < hi.
+    const uint64_t span = hi - lo;
+    const uint64_t mid = lo + (span < (1ull << 32) ? span * (lane + 1) / (kSplitLanes + 1)
+                                                   : span / (kSplitLanes + 1) * (lane + 1));
+    bool right = false;  // the split lies after mid
+    if (lo < hi) {
+      const E x{to_ordered(A[mid], xf), LEX ? to_ordered(AV[mid], vxf) : V(0)};
+      const uint64_t o = diag - 1 - mid;
+      const E y{to_ordered(B[o], xf), LEX ? to_ordered(BV[o], vxf) : V(0)};
+      right = x <= y;
+    }
+    // Lanes that say right come first; the next range lies between the last of
+    // them and the first that does not.
+    const uint32_t n = (uint32_t)__popcll((ballot(right) >> shift) & ((1u << kSplitLanes) - 1));
+    const uint32_t me = lane_id() - lane;
+    const uint64_t below = __shfl(mid, (int)(me + (n ? n - 1 : 0)));
+    const uint64_t above = __shfl(mid, (int)(me + (n < kSplitLanes ? n : kSplitLanes - 1)));
+    if (lo < hi) {
+      if (n < kSplitLanes) hi = above;
+      if (n) lo = below + 1;
+    }
+  }
+  if (in && lane == 0) a_split[t] = lo;
 }
 
+// What bounds it: LDS work and the reads in flight.  All of a thread's loads
+// are issued before any is staged, and the merge keeps the two heads in
+// registers: one LDS read an element.  2^25 + 2^24 u32 + u32 pairs: the call 245
+// -> 179 us (4.5 TB/s of keys and payloads read and written), of which the
+// tables that one job does not need any more were about 30.
 template <typename U, typename V, bool KV, bool LEX, int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void merge_tile_kernel(const U* __restrict__ ska, const U* __restrict__ skb,
                                                              const V* __restrict__ sva, const V* __restrict__ svb,
-                                                             U* __restrict__ dk, V* __restrict__ dv,
-                                                             const MergeJobDev* __restrict__ jobs,
-                                                             const uint32_t* __restrict__ tile_job,
+                                                             U* __restrict__ dk, V* __restrict__ dv, MergeJobs jobs,
                                                              const uint64_t* __restrict__ a_split, Xform<U> xf,
                                                              Xform<V> vxf) {
   using E = MKey<U, V, LEX>;
@@ -84,7 +125,7 @@ __global__ __launch_bounds__(THREADS) void merge_tile_kernel(const U* __restrict
 
   const uint32_t t = blockIdx.x;
   const uint32_t tid = threadIdx.x;
-  const MergeJobDev jb = jobs[tile_job[t]];
+  const MergeJobDev jb = jobs.of(t);
   const uint64_t L = jb.a_len + jb.b_len;
   const uint64_t d0 = (uint64_t)(t - jb.tile0) * TILE;
   const uint64_t d1 = (d0 + TILE < L) ? d0 + TILE : L;
@@ -95,35 +136,57 @@ __global__ __launch_bounds__(THREADS) void merge_tile_kernel(const U* __restrict
   const uint32_t tot = (uint32_t)(d1 - d0);
   const uint32_t nb = tot - na;
 
-  for (uint32_t i = tid; i < tot; i += THREADS) {
-    if (i < na) {
-      const uint64_t g = jb.a_off + a0 + i;
-      s_k[i] = to_ordered(ska[g], xf);
-      if constexpr (KV) s_v[i] = sva[g];
-    } else {
-      const uint64_t g = jb.b_off + b0 + (i - na);
-      s_k[i] = to_ordered(skb[g], xf);
-      if constexpr (KV) s_v[i] = svb[g];
+  {
+    const U* const ka = ska + jb.a_off + a0;
+    const U* const kb = skb + jb.b_off + b0;
+    const V* const va = sva + jb.a_off + a0;
+    const V* const vb = svb + jb.b_off + b0;
+    U k[ITEMS];
+    V v[KV ? ITEMS : 1];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      const uint32_t i = (uint32_t)j * THREADS + tid;
+      if (i < tot) {
+        k[j] = i < na ? ka[i] : kb[i - na];
+        if constexpr (KV) v[j] = i < na ? va[i] : vb[i - na];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      const uint32_t i = (uint32_t)j * THREADS + tid;
+      if (i < tot) {
+        s_k[i] = to_ordered(k[j], xf);
+        if constexpr (KV) s_v[i] = v[j];
+      }
     }
   }
-  __syncthreads();
+  lds_barrier();
 
   const uint32_t diag = (tid * ITEMS < tot) ? tid * ITEMS : tot;
   auto elem = [&](uint32_t i) { return E{s_k[i], LEX ? to_ordered(s_v[i], vxf) : V(0)}; };
   uint32_t ia = (uint32_t)merge_path_search<E>(
       diag, na, nb, [&](uint64_t i) { return elem((uint32_t)i); }, [&](uint64_t i) { return elem(na + (uint32_t)i); });
-  uint32_t ib = diag - ia;
+  // Positions of the two heads in the staged tile (a run's end reads a valid
+  // element that is not used).
+  uint32_t ib = na + diag - ia;
+  E ha = elem(ia < tot ? ia : tot - 1), hb = elem(ib < tot ? ib : tot - 1);
   U ok[ITEMS];
   uint32_t osrc[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     if (diag + k < tot) {
-      const bool take_a = ib >= nb || (ia < na && elem(ia) <= elem(na + ib));
-      const uint32_t src = take_a ? ia : na + ib;
-      ok[k] = s_k[src];
-      osrc[k] = src;
-      ia += take_a ? 1u : 0u;
-      ib += take_a ? 0u : 1u;
+      const bool take_a = ib >= tot || (ia < na && ha <= hb);
+      ok[k] = take_a ? ha.k : hb.k;
+      osrc[k] = take_a ? ia : ib;
+      const uint32_t next = (take_a ? ia : ib) + 1;
+      const E h = elem(next < tot ? next : tot - 1);
+      if (take_a) {
+        ia = next;
+        ha = h;
+      } else {
+        ib = next;
+        hb = h;
+      }
     }
   }
   V ov[KV ? ITEMS : 1];
@@ -132,7 +195,7 @@ __global__ __launch_bounds__(THREADS) void merge_tile_kernel(const U* __restrict
     for (int k = 0; k < ITEMS; ++k)
       if (diag + k < tot) ov[k] = s_v[osrc[k]];
   }
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     if (diag + k < tot) {
@@ -140,10 +203,14 @@ __global__ __launch_bounds__(THREADS) void merge_tile_kernel(const U* __restrict
       if constexpr (KV) s_v[diag + k] = ov[k];
     }
   }
-  __syncthreads();
-  for (uint32_t i = tid; i < tot; i += THREADS) {
-    dk[jb.out_off + d0 + i] = from_ordered(s_k[i], xf);
-    if constexpr (KV) dv[jb.out_off + d0 + i] = s_v[i];
+  lds_barrier();
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    const uint32_t i = (uint32_t)j * THREADS + tid;
+    if (i < tot) {
+      dk[jb.out_off + d0 + i] = from_ordered(s_k[i], xf);
+      if constexpr (KV) dv[jb.out_off + d0 + i] = s_v[i];
+    }
   }
 }
 
@@ -156,50 +223,56 @@ struct MValT<8> {
   using T = uint64_t;
 };
 
-constexpr int kMergeThreads = 256;
-constexpr int kMergeItems = 8;
 
-uint32_t merge_tile_elems() { return kMergeThreads * kMergeItems; }
+// 512 threads, an odd number of items (a thread's consecutive slots then spread
+// over the LDS banks): 13, where key and payload take 16 bytes 9 (two workgroups
+// a CU).  Merges of 50 M u32 + u32, 67 M u32, 33 M u64 + i64: 256 x 8 (with the
+// same loads and heads) 206, 209, 245 us; 512 x 9 183, 167, 240; 512 x 13 179,
+// 142, 303; 1024 x 9 199, 167, 269.
+constexpr int kMergeThreads = 512;
+constexpr int merge_items(int kb, int vb) { return kb + vb > 12 ? 9 : 13; }
+
+uint32_t merge_tile_elems(int kb, int vb) { return kMergeThreads * merge_items(kb, vb); }
 
 template <typename U, int VB, bool LEX>
 static hipError_t merge_launch(const void* ska, const void* skb, const void* sva, const void* svb, void* dk,
-                               void* dv, const MergeJobDev* d_jobs, const uint32_t* d_tile_job, uint32_t ntiles,
+                               void* dv, const MergeJobs& jobs, uint32_t ntiles,
                                const XformParams& xp, const XformParams& vp, uint64_t* d_split, hipStream_t stream) {
   using V = typename MValT<VB>::T;
   constexpr bool KV = VB != 0;
+  constexpr int ITEMS = merge_items(sizeof(U), VB);
   const Xform<U> xf{(U)xp.float_mask, (U)xp.sign_flip, (U)xp.desc_mask};
   const Xform<V> vxf{(V)vp.float_mask, (V)vp.sign_flip, (V)vp.desc_mask};
-  hipLaunchKernelGGL((merge_partition_kernel<U, V, LEX>), dim3((ntiles + 255) / 256), dim3(256), 0, stream,
+  hipLaunchKernelGGL((merge_partition_kernel<U, V, LEX>), dim3((uint32_t)(((uint64_t)ntiles * kSplitLanes + 255) / 256)),
+                     dim3(256), 0, stream,
                      reinterpret_cast<const U*>(ska), reinterpret_cast<const U*>(skb),
-                     reinterpret_cast<const V*>(sva), reinterpret_cast<const V*>(svb), d_jobs, d_tile_job, ntiles,
-                     merge_tile_elems(), xf, vxf, d_split);
-  hipLaunchKernelGGL((merge_tile_kernel<U, V, KV, LEX, kMergeThreads, kMergeItems>), dim3(ntiles),
+                     reinterpret_cast<const V*>(sva), reinterpret_cast<const V*>(svb), jobs, ntiles,
+                     (uint32_t)(kMergeThreads * ITEMS), xf, vxf, d_split);
+  hipLaunchKernelGGL((merge_tile_kernel<U, V, KV, LEX, kMergeThreads, ITEMS>), dim3(ntiles),
                      dim3(kMergeThreads), 0, stream, reinterpret_cast<const U*>(ska), reinterpret_cast<const U*>(skb),
                      reinterpret_cast<const V*>(sva), reinterpret_cast<const V*>(svb), reinterpret_cast<U*>(dk),
-                     reinterpret_cast<V*>(dv), d_jobs, d_tile_job, d_split, xf, vxf);
+                     reinterpret_cast<V*>(dv), jobs, d_split, xf, vxf);
   return hipGetLastError();
 }
 
-hipError_t merge_tiles(int kb, int vb, const void* ska, const void* skb, const void* sva, const void* svb, void* dk,
-                       void* dv, const MergeJobDev* d_jobs, const uint32_t* d_tile_job, uint32_t ntiles,
-                       const XformParams& xf, uint64_t* d_split, hipStream_t stream, const XformParams* lex_vxf) {
+static hipError_t merge_any(int kb, int vb, const void* ska, const void* skb, const void* sva, const void* svb,
+                            void* dk, void* dv, const MergeJobs& jobs, uint32_t ntiles, const XformParams& xf,
+                            uint64_t* d_split, hipStream_t stream, const XformParams* lex_vxf) {
   if (ntiles == 0) return hipSuccess;
   const XformParams vz{0, 0, 0};
   const bool lex = lex_vxf != nullptr && vb != 0;
   const XformParams& vp = lex ? *lex_vxf : vz;
-#define GS_MERGE_CASE(UT, VBV)                                                                                    \
-  return lex ? merge_launch<UT, VBV, true>(ska, skb, sva, svb, dk, dv, d_jobs, d_tile_job, ntiles, xf, vp, d_split, \
-                                           stream)                                                                \
-             : merge_launch<UT, VBV, false>(ska, skb, sva, svb, dk, dv, d_jobs, d_tile_job, ntiles, xf, vp,       \
-                                            d_split, stream)
+#define GS_MERGE_CASE(UT, VBV)                                                                              \
+  return lex ? merge_launch<UT, VBV, true>(ska, skb, sva, svb, dk, dv, jobs, ntiles, xf, vp, d_split, stream) \
+             : merge_launch<UT, VBV, false>(ska, skb, sva, svb, dk, dv, jobs, ntiles, xf, vp, d_split, stream)
   if (kb == 4) {
-    if (vb == 0) return merge_launch<uint32_t, 0, false>(ska, skb, sva, svb, dk, dv, d_jobs, d_tile_job, ntiles, xf, vp,
-                                                         d_split, stream);
+    if (vb == 0)
+      return merge_launch<uint32_t, 0, false>(ska, skb, sva, svb, dk, dv, jobs, ntiles, xf, vp, d_split, stream);
     if (vb == 4) GS_MERGE_CASE(uint32_t, 4);
     if (vb == 8) GS_MERGE_CASE(uint32_t, 8);
   } else if (kb == 8) {
-    if (vb == 0) return merge_launch<uint64_t, 0, false>(ska, skb, sva, svb, dk, dv, d_jobs, d_tile_job, ntiles, xf, vp,
-                                                         d_split, stream);
+    if (vb == 0)
+      return merge_launch<uint64_t, 0, false>(ska, skb, sva, svb, dk, dv, jobs, ntiles, xf, vp, d_split, stream);
     if (vb == 4) GS_MERGE_CASE(uint64_t, 4);
     if (vb == 8) GS_MERGE_CASE(uint64_t, 8);
   }
@@ -207,8 +280,25 @@ hipError_t merge_tiles(int kb, int vb, const void* ska, const void* skb, const v
   return hipErrorInvalidValue;
 }
 
-// Host-side tiling of a job list: fills the device job records and the
-// tile -> job table.  Returns the number of tiles.
+hipError_t merge_tiles(int kb, int vb, const void* ska, const void* skb, const void* sva, const void* svb, void* dk,
+                       void* dv, const MergeJobDev* d_jobs, const uint32_t* d_tile_job, uint32_t ntiles,
+                       const XformParams& xf, uint64_t* d_split, hipStream_t stream, const XformParams* lex_vxf) {
+  return merge_any(kb, vb, ska, skb, sva, svb, dk, dv, MergeJobs{d_jobs, d_tile_job, {}}, ntiles, xf, d_split, stream,
+                   lex_vxf);
+}
+
+uint64_t merge_two_tiles(int kb, int vb, uint64_t n) {
+  const uint64_t tile = merge_tile_elems(kb, vb);
+  return (n + tile - 1) / tile;
+}
+
+hipError_t merge_two(int kb, int vb, const void* a_k, const void* a_v, uint64_t na, const void* b_k, const void* b_v,
+                     uint64_t nb, void* dk, void* dv, const XformParams& xf, uint64_t* d_split, hipStream_t stream) {
+  const MergeJobs jobs{nullptr, nullptr, MergeJobDev{0, na, 0, nb, 0, 0, 0}};
+  return merge_any(kb, vb, a_k, b_k, a_v, b_v, dk, dv, jobs, (uint32_t)merge_two_tiles(kb, vb, na + nb), xf, d_split,
+                   stream, nullptr);
+}
+
 // ------------------------------------------------------ bitonic merge-split cuts
 //
 // One merge-split of SampleSort's small-input bitonic network keeps a prefix
@@ -335,8 +425,11 @@ hipError_t net_cuts(int kb, int vb, const void* keys, const void* vals, const Ne
   return hipErrorInvalidValue;
 }
 
-uint32_t merge_plan(const MergeJob* jobs, uint32_t njobs, MergeJobDev* out_jobs, std::vector<uint32_t>* tile_job) {
-  const uint32_t T = merge_tile_elems();
+// Host-side tiling of a job list: fills the device job records and the
+// tile -> job table.  Returns the number of tiles.
+uint32_t merge_plan(int kb, int vb, const MergeJob* jobs, uint32_t njobs, MergeJobDev* out_jobs,
+                    std::vector<uint32_t>* tile_job) {
+  const uint32_t T = merge_tile_elems(kb, vb);
   tile_job->clear();
   for (uint32_t j = 0; j < njobs; ++j) {
     const uint64_t L = jobs[j].a_len + jobs[j].b_len;

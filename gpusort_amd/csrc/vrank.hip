@@ -204,7 +204,7 @@ struct Run {
 gs_status run_merge_jobs(Pipe& P, const std::vector<MergeJob>& jobs) {
   std::vector<MergeJobDev> dj(jobs.size());
   std::vector<uint32_t> tile_job;
-  const uint32_t ntiles = merge_plan(jobs.data(), (uint32_t)jobs.size(), dj.data(), &tile_job);
+  const uint32_t ntiles = merge_plan(P.kb, P.kv ? P.vb : 0, jobs.data(), (uint32_t)jobs.size(), dj.data(), &tile_job);
   if (ntiles) {
     AuxLayout L;
     const size_t o_j = L.add(dj.data(), dj.size() * sizeof(MergeJobDev));
