@@ -70,10 +70,14 @@ uint32_t block_sort_max(int kb, int vb) {
 
 uint32_t block_sort_tile_max(int kb, int vb) { return 1024u * (uint32_t)wide_items(kb, vb); }
 
+uint32_t block_sort_class_len(int kb, int vb, int cls) {
+  return cls < 3 ? kClassLen[cls] : 512u * (uint32_t)wide_items(kb, vb);
+}
+
 int block_sort_class(int kb, int vb, uint32_t len) {
-  for (int c = 0; c < 3; ++c)
-    if (len <= kClassLen[c]) return c;
-  return len <= 512u * (uint32_t)wide_items(kb, vb) ? 3 : 4;
+  for (int c = 0; c < kBlockClasses - 1; ++c)
+    if (len <= block_sort_class_len(kb, vb, c)) return c;
+  return kBlockClasses - 1;
 }
 
 template <int VB>

@@ -93,6 +93,33 @@ void Arena::release() {
   }
 }
 
+// ---------------------------------------------------------------- stage
+void* PinnedStage::take(size_t bytes, hipStream_t stream) {
+  bytes = align_up(bytes ? bytes : 1, 256);
+  if (bytes > kBytes || failed_) return nullptr;
+  if (!base_) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kBytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      failed_ = true;
+      return nullptr;
+    }
+    base_ = static_cast<char*>(p);
+  }
+  if (used_ + bytes > kBytes) {
+    if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
+    used_ = 0;
+  }
+  used_ += bytes;
+  return base_ + used_ - bytes;
+}
+
+void PinnedStage::release() {
+  if (base_) (void)hipHostFree(base_);
+  base_ = nullptr;
+  used_ = 0;
+}
+
 // ---------------------------------------------------------------- profiler
 Profiler::~Profiler() {
   for (hipEvent_t e : pool_) (void)hipEventDestroy(e);
@@ -441,6 +468,7 @@ gs_status gs_destroy(gs_handle* h) {
     (void)hipStreamSynchronize(h->stream);
     h->arena.release();
     if (h->pinned) (void)hipHostFree(h->pinned);
+    h->stage.release();
     if (h->gather_done) (void)hipEventDestroy(h->gather_done);
   }
   delete h;

@@ -67,6 +67,25 @@ class Arena {
   size_t cap_[kSlots];
 };
 
+// Pinned host memory for the small transfers of a call (plans and offset
+// tables up, samples and bounds down): copies through it return at once, where
+// one from pageable memory takes 10-20 us of the host's time and the wait that
+// its source needs.  Handed out front to back; when it is used up the stream is
+// drained and it starts over.
+class PinnedStage {
+ public:
+  static constexpr size_t kBytes = 4u << 20;
+  // Room for `bytes`, or null (too large, or no pinned memory): the caller then
+  // copies from and to its own memory.
+  void* take(size_t bytes, hipStream_t stream);
+  void release();
+
+ private:
+  char* base_ = nullptr;
+  size_t used_ = 0;
+  bool failed_ = false;
+};
+
 class DeviceScope {
  public:
   explicit DeviceScope(int dev);
@@ -117,6 +136,8 @@ struct gs_handle {
   gs::LaunchTimer* timer() { return profiler.active ? &profiler : nullptr; }
   void* pinned = nullptr;
   size_t pinned_bytes = 0;
+  gs::PinnedStage stage;
+  std::vector<uint64_t> seg_offsets;  // gs_sort_segments' host copy
   // Size-class configuration of the batched sort per (key, payload) width,
   // set by the autotuner; defaults otherwise.
   std::map<int, gs::SegConfig> seg_tuned;

@@ -143,6 +143,8 @@ hipError_t block_sort(int key_bytes, int val_bytes, void* keys, void* vals, uint
 // and its LDS tile grow with the class); longer ones are left untouched.
 constexpr int kBlockClasses = 5;
 int block_sort_class(int key_bytes, int val_bytes, uint32_t len);
+// The longest segment of a class but the last.
+uint32_t block_sort_class_len(int key_bytes, int val_bytes, int cls);
 hipError_t block_sort_segments(int key_bytes, int val_bytes, void* keys, void* vals, const uint64_t* d_offsets,
                                const uint32_t* d_seg_ids, uint32_t nblocks, const XformParams& xf,
                                hipStream_t stream, int cls);

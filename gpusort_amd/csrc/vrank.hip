@@ -39,6 +39,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <vector>
 
 #include "../../include/gpusort_hip.h"
@@ -59,11 +60,32 @@ struct Pipe {
   char* vbuf[2];
   int cur;
   uint64_t n;
-  // host-side aux staging (device copies live in the aux arena slot)
-  std::vector<char> stage;
-  // host sources of queued uploads, kept until the call's final wait
+  // host sources of queued uploads that did not fit the handle's pinned stage,
+  // kept until the call's final wait
   std::vector<std::vector<unsigned char>> keep;
 };
+
+// Copies blocks of device memory to host memory, and waits for them.
+struct ReadBlock {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+
+hipError_t read_blocks(Pipe& P, std::initializer_list<ReadBlock> blocks) {
+  std::vector<std::pair<const ReadBlock*, void*>> staged;
+  for (const ReadBlock& b : blocks) {
+    if (b.bytes == 0) continue;
+    void* at = P.h->stage.take(b.bytes, P.h->stream);
+    if (at) staged.push_back({&b, at});
+    const hipError_t e = hipMemcpyAsync(at ? at : b.dst, b.src, b.bytes, hipMemcpyDeviceToHost, P.h->stream);
+    if (e != hipSuccess) return e;
+  }
+  const hipError_t e = hipStreamSynchronize(P.h->stream);
+  if (e != hipSuccess) return e;
+  for (const auto& s : staged) memcpy(s.first->dst, s.second, s.first->bytes);
+  return hipSuccess;
+}
 
 bool is_pow2(uint64_t x) { return x && !(x & (x - 1)); }
 
@@ -96,7 +118,7 @@ gs_status sort_runs(Pipe& P, char* k, char* v, const std::vector<uint64_t>& off,
                        P.desc);
       if (st != GS_OK) return st;
     }
-    // `meta` is the source of an upload queued above: kept until the end.
+    // `meta`, if not empty, is the source of an upload queued above: kept until the end.
     P.keep.push_back(std::move(meta));
     return GS_OK;
   };
@@ -129,11 +151,14 @@ gs_status upload(Pipe& P, AuxLayout& L, char** base, size_t scratch = 0) {
   hipError_t e = P.h->arena.get(Arena::kPipeAux, L.total + scratch, P.h->stream, &ws);
   if (e != hipSuccess) return from_hip(e, "pipeline workspace");
   *base = reinterpret_cast<char*>(ws);
-  P.stage.assign(L.total, 0);
+  char* stage = reinterpret_cast<char*>(P.h->stage.take(L.total, P.h->stream));
+  if (!stage) {
+    P.keep.emplace_back(L.total);
+    stage = reinterpret_cast<char*>(P.keep.back().data());
+  }
   for (size_t i = 0; i < L.blocks.size(); ++i)
-    if (L.blocks[i].first && L.blocks[i].second) memcpy(P.stage.data() + L.offs[i], L.blocks[i].first, L.blocks[i].second);
-  e = hipMemcpyAsync(ws, P.stage.data(), L.total, hipMemcpyHostToDevice, P.h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(P.h->stream);  // stage buffer is reused by the next upload
+    if (L.blocks[i].first && L.blocks[i].second) memcpy(stage + L.offs[i], L.blocks[i].first, L.blocks[i].second);
+  e = hipMemcpyAsync(ws, stage, L.total, hipMemcpyHostToDevice, P.h->stream);
   return from_hip(e, "pipeline upload");
 }
 
@@ -162,10 +187,7 @@ gs_status gather_sorted(Pipe& P, const std::vector<uint64_t>& idx, const std::ve
     st = sort_segment(P, base + o_k + a * P.kb, P.kv ? base + o_v + a * P.vb : nullptr, b - a, P.kv);
     if (st != GS_OK) return st;
   }
-  e = hipMemcpyAsync(hk->data(), base + o_k, (size_t)m * P.kb, hipMemcpyDeviceToHost, P.h->stream);
-  if (e == hipSuccess && P.kv)
-    e = hipMemcpyAsync(hv->data(), base + o_v, (size_t)m * P.vb, hipMemcpyDeviceToHost, P.h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(P.h->stream);
+  e = read_blocks(P, {{hk->data(), base + o_k, (size_t)m * P.kb}, {hv->data(), base + o_v, hv->size()}});
   return from_hip(e, "read samples");
 }
 
@@ -189,9 +211,7 @@ gs_status run_bounds(Pipe& P, const std::vector<uint64_t>& off, const std::vecto
                                reinterpret_cast<const uint32_t*>(base + o_first), nspl, upper ? 1 : 0, P.kx,
                                reinterpret_cast<uint64_t*>(base + o_b), P.h->stream, P.kv ? P.vb : 0,
                                P.kv ? P.vbuf[P.cur] : nullptr, P.kv ? base + o_sv : nullptr, P.kv ? &P.vx : nullptr);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(bounds->data(), base + o_b, bounds->size() * 8, hipMemcpyDeviceToHost, P.h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(P.h->stream);
+  if (e == hipSuccess) e = read_blocks(P, {{bounds->data(), base + o_b, bounds->size() * 8}});
   return from_hip(e, "bucket bounds");
 }
 
@@ -219,7 +239,6 @@ gs_status run_merge_jobs(Pipe& P, const std::vector<MergeJob>& jobs) {
                                reinterpret_cast<const MergeJobDev*>(base + o_j),
                                reinterpret_cast<const uint32_t*>(base + o_t), ntiles, P.kx,
                                reinterpret_cast<uint64_t*>(base + o_s), P.h->stream, P.kv ? &P.vx : nullptr);
-    if (e == hipSuccess) e = hipStreamSynchronize(P.h->stream);
     if (e != hipSuccess) return from_hip(e, "merge level");
   }
   P.cur ^= 1;
@@ -288,7 +307,6 @@ gs_status merge_lists(Pipe& P, std::vector<std::vector<Run>> lists, const std::v
     hipError_t e = kway_merge(P.kb, vb, P.kbuf[src], P.kv ? P.vbuf[src] : nullptr, P.kbuf[dst],
                               P.kv ? P.vbuf[dst] : nullptr, plan.totals, dev, P.kx, P.kv ? &P.vx : nullptr,
                               P.h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(P.h->stream);
     if (e != hipSuccess) return from_hip(e, "k-way merge");
     P.cur ^= 1;
     lists.swap(next);
@@ -542,9 +560,7 @@ gs_status samplesort_small(Pipe& P, std::vector<uint64_t>& sizes, uint32_t* roun
     hipError_t e = net_cuts(P.kb, P.kv ? P.vb : 0, P.kbuf[P.cur], P.kv ? P.vbuf[P.cur] : nullptr,
                             reinterpret_cast<const NetCut*>(base + o_ops), nops, P.kx, P.kv ? &P.vx : nullptr,
                             P.desc ? 0 : 1, reinterpret_cast<NetCutResult*>(base + o_out), P.h->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(res.data(), base + o_out, nops * sizeof(NetCutResult), hipMemcpyDeviceToHost, P.h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(P.h->stream);
+    if (e == hipSuccess) e = read_blocks(P, {{res.data(), base + o_out, nops * sizeof(NetCutResult)}});
     if (e != hipSuccess) return from_hip(e, "bitonic cuts");
     std::vector<uint64_t> ns = sizes;
     std::vector<bool> busy(p, false);
