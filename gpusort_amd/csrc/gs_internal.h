@@ -27,16 +27,16 @@ XformParams make_xform(int kind, bool descending);
 
 constexpr int kMaxPasses = 8;
 constexpr uint32_t kSkipPass = 0xFFFFFFFFu;
+constexpr uint32_t kCopyPass = 4;  // a pass that only copies from buffer (src & 1) to the other one
 
 // Device-resident control block of one radix sort: which ping-pong buffer
 // each pass reads (decided on the device from the digit histograms, so no
-// host round trip is needed), the tile tickets of each pass, and the buffer
-// that holds the result.
+// host round trip is needed; the result lands where the keys were), and the
+// tile tickets of each pass.
 struct SortCtrl {
   uint32_t src[kMaxPasses];
   uint32_t tile_counter[kMaxPasses];
-  uint32_t final_sel;
-  uint32_t passes_run;
+  uint32_t unused[2];
   // Tile tickets per workgroup class (blockIdx % 8) when a pass hands out
   // tiles in XCD groups.
   uint32_t class_counter[kMaxPasses][8];
@@ -72,7 +72,10 @@ enum TilePolicy : int { kTilesByStream = -1, kTilesArrival = 0, kTilesGrouped = 
 // Onesweep LSD radix sort of n keys (key_bytes 4/8) with an optional payload
 // (val_bytes 0/4/8), stable.  keys/vals are sorted in place; the workspace
 // holds the ping-pong buffers, histograms and look-back status words.
+// radix_workspace_min_bytes: the least it can do with (larger tiles than it
+// would choose).
 size_t radix_workspace_bytes(int key_bytes, int val_bytes, uint64_t n);
+size_t radix_workspace_min_bytes(int key_bytes, int val_bytes, uint64_t n);
 hipError_t radix_sort(int key_bytes, int val_bytes, void* keys, void* vals, uint64_t n, const XformParams& xf,
                       void* workspace, size_t workspace_bytes, hipStream_t stream, LaunchTimer* timer = nullptr,
                       int tile_policy = kTilesByStream);

@@ -65,7 +65,7 @@ extern "C" gs_status gs_sort_pairs_noalloc(gs_handle* h, gs_dtype kdt, void* d_k
   const XformParams xf = make_xform((int)kdt, descending != 0);
   if (n <= block_sort_tile_max(kb, vb))  // one workgroup in LDS: no workspace
     return from_hip(block_sort(kb, vb, d_keys, d_vals, (uint32_t)n, xf, h->stream), "block sort");
-  const size_t need = radix_workspace_bytes(kb, vb, n);
+  const size_t need = radix_workspace_min_bytes(kb, vb, n);
   if (need > (size_t)GS_NOALLOC_SCRATCH_BYTES)
     return fail(GS_INVALID_ARG,
                 "gs_sort_pairs_noalloc: %llu keys of %d + %d bytes need %zu bytes of workspace, more than the "

@@ -4,7 +4,7 @@
 //   thrust::sort         (src/cuda_utils.cu:424)       -- keys only
 //   thrust::sort_by_key  (src/cuda_utils.cu:477-478)   -- stable, with payload
 //
-// One sort is 3 + P launches on one stream, with no host synchronisation:
+// One sort is 3 + P launches (two more for 64-bit keys) on one stream, with no host synchronisation:
 //   prep      zero the global digit histograms; 64-bit keys: pick the lowest
 //             digit to sort by from a sample (radix_ties.h)
 //   hist      one read of all keys -> the 256-bin histogram of every digit
@@ -14,7 +14,8 @@
 //             every remaining pass is chosen on the device
 //   pass x P  onesweep pass (below)
 //   ties      64-bit keys: two launches that order what the passes left
-//   copy      only if the result ended in the temporary buffer
+//             (where an odd number of passes is to run, one of those left out
+//             copies instead, so that the result lands where the keys were)
 //
 // Onesweep pass, per tile of THREADS*ITEMS keys (tile order from an atomic
 // ticket per workgroup class so every tile's predecessors are already
@@ -282,18 +283,19 @@ __global__ __launch_bounds__(256) void radix_scan_kernel(const unsigned long lon
   }
   __syncthreads();
   if (tid < kMaxPasses) {
-    uint32_t before = 0, run = 0;  // passes that run before this one, and in all
-    for (uint32_t p = 0; p < kMaxPasses; ++p) {
-      const uint32_t r = s_trivial[p] ? 0u : 1u;
-      before += p < tid ? r : 0u;
-      run += r;
+    // An odd number of passes would leave the result in the other buffer: the
+    // first pass that is left out then copies (an even number of digits, so
+    // there is one).
+    uint32_t run = 0, copy = kMaxPasses;
+    for (uint32_t p = 0; p < (uint32_t)passes; ++p) {
+      run += s_trivial[p] ? 0u : 1u;
+      if (s_trivial[p] && copy == kMaxPasses) copy = p;
     }
+    if (!(run & 1u)) copy = kMaxPasses;
+    uint32_t before = 0;
+    for (uint32_t p = 0; p < tid; ++p) before += (s_trivial[p] && p != copy) ? 0u : 1u;
     ctrl->tile_counter[tid] = 0;
-    ctrl->src[tid] = s_trivial[tid] ? kSkipPass : (before & 1u);
-    if (tid == 0) {
-      ctrl->final_sel = run & 1u;
-      ctrl->passes_run = run;
-    }
+    ctrl->src[tid] = tid == copy ? (kCopyPass | (before & 1u)) : s_trivial[tid] ? kSkipPass : (before & 1u);
   }
 }
 
@@ -565,7 +567,20 @@ __global__ __launch_bounds__(THREADS) void onesweep_kernel(OnesweepArgs<U, V, S>
     src = (uint32_t)a.pass & 1u;
   } else {
     src = a.ctrl->src[a.pass];
-    if (src > 1u) return;  // every key has the same digit here: the pass is the identity
+    if (src > 1u) {  // every key has the same digit here: the pass is the identity
+      if (src != kSkipPass) {
+        const uint64_t end = (uint64_t)(blockIdx.x + 1) * TILE < a.n ? (uint64_t)(blockIdx.x + 1) * TILE : a.n;
+        const U* const kc = (src & 1u) ? a.keys1 : a.keys0;
+        U* const kd = (src & 1u) ? a.keys0 : a.keys1;
+        const V* const vc = (src & 1u) ? a.vals1 : a.vals0;
+        V* const vd = (src & 1u) ? a.vals0 : a.vals1;
+        for (uint64_t i = (uint64_t)blockIdx.x * TILE + threadIdx.x; i < end; i += THREADS) {
+          kd[i] = kc[i];
+          if constexpr (KV) vd[i] = vc[i];
+        }
+      }
+      return;
+    }
   }
   const U* __restrict__ kin = src ? a.keys1 : a.keys0;
   U* __restrict__ kout = src ? a.keys0 : a.keys1;
@@ -868,18 +883,6 @@ __global__ __launch_bounds__(THREADS) void onesweep_kernel(OnesweepArgs<U, V, S>
     tile_body(std::false_type{});
 }
 
-template <typename U, typename V, bool KV>
-__global__ __launch_bounds__(256) void radix_final_copy_kernel(U* __restrict__ k0, const U* __restrict__ k1,
-                                                               V* __restrict__ v0, const V* __restrict__ v1,
-                                                               uint64_t n, const SortCtrl* ctrl) {
-  if (ctrl->final_sel == 0) return;
-  const uint64_t stride = (uint64_t)gridDim.x * 256;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-    k0[i] = k1[i];
-    if constexpr (KV) v0[i] = v1[i];
-  }
-}
-
 // ------------------------------------------------------------------ host side
 
 template <typename U, int VB>
@@ -916,31 +919,73 @@ struct Geometry<uint64_t, 8> {
   static constexpr int THREADS = 1024, ITEMS = 9;
 };
 
-// Smaller tiles for mid-size single arrays, where the large tile leaves CUs
-// idle (2^22 keys-only 32-bit keys are 137 tiles of 30 K for 256 CUs):
-// keys-only 32-bit keys up to 2^23 keys at 1024 x 16, 32-bit keys with
-// 32-bit payloads up to 2^21 keys at 1024 x 10, keys-only 64-bit keys up to
-// 2^21 keys at 1024 x 8.  MAX_N 0: no smaller tile.
+// Tiles of a single-array sort, the large one first.  A pass takes a round of
+// tiles a CU (one workgroup each), so an array whose last round is nearly empty
+// does better with the smallest tile that needs no more rounds, and one of a
+// few tiles with a small workgroup: 16.8 M u32 keys 283 us with 30 items, 267
+// with 22; 5.5 M 149 (16 items) -> 116 (22); 3 M u32 + u32 112 (19) -> 106 (13);
+// 60,000 u32 + u32 54 (1024 x 10) -> 47 (512 x 8), 250,000 u64 + u32 93 (1024 x
+// 13) -> 81, u32 + i64 69 -> 57.  Past max_rounds the larger
+// tile's shorter look-back weighs more (12 M u32 + u32: 279 with 19, 283 with
+// 16; 67 M 1247, 1261); up to tiny_max the last one is taken.
+struct SortTile {
+  int threads, items;
+};
 template <typename U, int VB>
-struct SmallGeometry {
-  static constexpr int THREADS = Geometry<U, VB>::THREADS, ITEMS = Geometry<U, VB>::ITEMS;
-  static constexpr uint64_t MAX_N = 0;
+struct SortTiles;
+template <>
+struct SortTiles<uint32_t, 0> {
+  static constexpr SortTile list[] = {{1024, 30}, {1024, 26}, {1024, 22}, {1024, 16}, {512, 12}};
+  static constexpr uint64_t tiny_max = 1ull << 20, max_rounds = 4;
 };
 template <>
-struct SmallGeometry<uint32_t, 0> {
-  static constexpr int THREADS = 1024, ITEMS = 16;
-  static constexpr uint64_t MAX_N = 1ull << 23;
+struct SortTiles<uint32_t, 4> {
+  static constexpr SortTile list[] = {{1024, 19}, {1024, 16}, {1024, 13}, {1024, 10}, {512, 8}};
+  static constexpr uint64_t tiny_max = 3ull << 17, max_rounds = 2;
 };
 template <>
-struct SmallGeometry<uint32_t, 4> {
-  static constexpr int THREADS = 1024, ITEMS = 10;
-  static constexpr uint64_t MAX_N = 1ull << 21;
+struct SortTiles<uint32_t, 8> {
+  static constexpr SortTile list[] = {{1024, 13}, {512, 8}};
+  static constexpr uint64_t tiny_max = 1ull << 20, max_rounds = 2;
 };
 template <>
-struct SmallGeometry<uint64_t, 0> {
-  static constexpr int THREADS = 1024, ITEMS = 8;
-  static constexpr uint64_t MAX_N = 1ull << 21;
+struct SortTiles<uint64_t, 0> {
+  static constexpr SortTile list[] = {{1024, 16}, {1024, 8}, {512, 8}};
+  static constexpr uint64_t tiny_max = 1ull << 18, max_rounds = 1;
 };
+template <>
+struct SortTiles<uint64_t, 4> {
+  static constexpr SortTile list[] = {{1024, 13}, {512, 8}};
+  static constexpr uint64_t tiny_max = 1ull << 20, max_rounds = 2;
+};
+template <>
+struct SortTiles<uint64_t, 8> {
+  static constexpr SortTile list[] = {{1024, 9}, {512, 8}};
+  static constexpr uint64_t tiny_max = 1ull << 19, max_rounds = 2;
+};
+template <typename U, int VB>
+constexpr int kSortTiles = sizeof(SortTiles<U, VB>::list) / sizeof(SortTile);
+
+constexpr uint64_t kRoundTiles = 256;  // one workgroup a CU
+
+// Which of its tiles a sort of n keys takes.
+template <typename U, int VB>
+static int sort_tile_of(uint64_t n) {
+  using T = SortTiles<U, VB>;
+  constexpr int last = kSortTiles<U, VB> - 1;
+  static_assert(T::list[0].threads == Geometry<U, VB>::THREADS && T::list[0].items == Geometry<U, VB>::ITEMS,
+                "the large tile first");
+  if (n <= T::tiny_max) return last;
+  auto rounds = [&](int i) {
+    const uint64_t keys = kRoundTiles * (uint64_t)T::list[i].threads * (uint64_t)T::list[i].items;
+    return (n + keys - 1) / keys;
+  };
+  int best = 0;
+  if (rounds(0) <= T::max_rounds)
+    for (int i = 1; i < last; ++i)
+      if (rounds(i) == rounds(0)) best = i;
+  return best;
+}
 
 template <int VB>
 struct ValT {
@@ -1048,20 +1093,25 @@ struct RadixLayout {
   size_t status_word;
 };
 
-// Tile of a single-array sort of n keys (SmallGeometry up to its MAX_N).
-static inline uint32_t sort_tile_keys(int kb, int vb, uint64_t n) {
-  if (kb == 4 && vb == 0 && n <= SmallGeometry<uint32_t, 0>::MAX_N)
-    return SmallGeometry<uint32_t, 0>::THREADS * SmallGeometry<uint32_t, 0>::ITEMS;
-  if (kb == 4 && vb == 4 && n <= SmallGeometry<uint32_t, 4>::MAX_N)
-    return SmallGeometry<uint32_t, 4>::THREADS * SmallGeometry<uint32_t, 4>::ITEMS;
-  if (kb == 8 && vb == 0 && n <= SmallGeometry<uint64_t, 0>::MAX_N)
-    return SmallGeometry<uint64_t, 0>::THREADS * SmallGeometry<uint64_t, 0>::ITEMS;
-  return tile_keys_for(kb, vb);
+// Keys a tile of a single-array sort of n keys holds (wide: the large tile,
+// whatever n, which needs the least workspace).
+template <typename U, int VB>
+static uint32_t sort_tile_keys_t(uint64_t n, bool wide) {
+  const SortTile t = SortTiles<U, VB>::list[wide ? 0 : sort_tile_of<U, VB>(n)];
+  return (uint32_t)(t.threads * t.items);
+}
+static uint32_t sort_tile_keys(int kb, int vb, uint64_t n, bool wide) {
+  if (kb == 4) {
+    if (vb == 0) return sort_tile_keys_t<uint32_t, 0>(n, wide);
+    return vb == 4 ? sort_tile_keys_t<uint32_t, 4>(n, wide) : sort_tile_keys_t<uint32_t, 8>(n, wide);
+  }
+  if (vb == 0) return sort_tile_keys_t<uint64_t, 0>(n, wide);
+  return vb == 4 ? sort_tile_keys_t<uint64_t, 4>(n, wide) : sort_tile_keys_t<uint64_t, 8>(n, wide);
 }
 
-static RadixLayout radix_layout(int kb, int vb, uint64_t n) {
+static RadixLayout radix_layout(int kb, int vb, uint64_t n, bool wide) {
   RadixLayout L{};
-  const uint32_t tile = sort_tile_keys(kb, vb, n);
+  const uint32_t tile = sort_tile_keys(kb, vb, n, wide);
   L.tiles = (n + tile - 1) / tile;
   L.passes = kb;  // 8-bit digits: one pass per key byte
   L.status_word = (n < (1ull << 30)) ? 4 : 8;
@@ -1083,7 +1133,10 @@ static RadixLayout radix_layout(int kb, int vb, uint64_t n) {
 }
 
 size_t radix_workspace_bytes(int key_bytes, int val_bytes, uint64_t n) {
-  return radix_layout(key_bytes, val_bytes, n).total;
+  return radix_layout(key_bytes, val_bytes, n, false).total;
+}
+size_t radix_workspace_min_bytes(int key_bytes, int val_bytes, uint64_t n) {
+  return radix_layout(key_bytes, val_bytes, n, true).total;
 }
 
 template <typename U>
@@ -1211,41 +1264,49 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
     t.tile_keys = n <= (1ull << 23) ? kTieChunk : 4 * kTieChunk;
     launch_tie_fix<V, KV>(t, (n + t.tile_keys - 1) / t.tile_keys, n, stream, timer);
   }
-  uint64_t copy_blocks = (n + 255) / 256;
-  if (copy_blocks > 1024) copy_blocks = 1024;  // reads one word and leaves where no copy is due
-  hipLaunchKernelGGL((radix_final_copy_kernel<U, V, KV>), dim3((uint32_t)copy_blocks), dim3(256), 0, stream, keys,
-                     keys_tmp, vals, vals_tmp, n, ctrl);
   return hipGetLastError();
 }
 
-template <typename U, int VB>
-static hipError_t radix_sort_s(U* keys, void* vals, uint64_t n, const XformParams& xp, unsigned char* ws,
+// The launch sequence of tile `tile` of the list.
+template <typename U, int VB, int I = 0>
+static hipError_t radix_sort_s(int tile, U* keys, void* vals, uint64_t n, const XformParams& xp, unsigned char* ws,
                                const RadixLayout& L, hipStream_t stream, LaunchTimer* timer, int policy) {
-  using G = Geometry<U, VB>;
-  using SG = SmallGeometry<U, VB>;
-  if (n <= SG::MAX_N)  // n < 2^30: 32-bit status words
-    return radix_sort_t<U, VB, uint32_t, SG::THREADS, SG::ITEMS>(keys, vals, n, xp, ws, L, stream, timer, policy);
-  if (L.status_word == 4)
-    return radix_sort_t<U, VB, uint32_t, G::THREADS, G::ITEMS>(keys, vals, n, xp, ws, L, stream, timer, policy);
-  return radix_sort_t<U, VB, uint64_t, G::THREADS, G::ITEMS>(keys, vals, n, xp, ws, L, stream, timer, policy);
+  constexpr SortTile T = SortTiles<U, VB>::list[I];
+  if constexpr (I == 0) {
+    if (L.status_word != 4)
+      return radix_sort_t<U, VB, uint64_t, T.threads, T.items>(keys, vals, n, xp, ws, L, stream, timer, policy);
+  }
+  if (tile == I)
+    return radix_sort_t<U, VB, uint32_t, T.threads, T.items>(keys, vals, n, xp, ws, L, stream, timer, policy);
+  if constexpr (I + 1 < kSortTiles<U, VB>)
+    return radix_sort_s<U, VB, I + 1>(tile, keys, vals, n, xp, ws, L, stream, timer, policy);
+  return hipErrorInvalidValue;
+}
+
+template <typename U, int VB>
+static hipError_t radix_sort_v(U* keys, void* vals, uint64_t n, const XformParams& xp, unsigned char* ws,
+                               const RadixLayout& L, bool wide, hipStream_t stream, LaunchTimer* timer, int policy) {
+  return radix_sort_s<U, VB>(wide ? 0 : sort_tile_of<U, VB>(n), keys, vals, n, xp, ws, L, stream, timer, policy);
 }
 
 hipError_t radix_sort(int kb, int vb, void* keys, void* vals, uint64_t n, const XformParams& xf, void* workspace,
                       size_t workspace_bytes, hipStream_t stream, LaunchTimer* timer, int policy) {
   if (n == 0) return hipSuccess;
-  const RadixLayout L = radix_layout(kb, vb, n);
+  RadixLayout L = radix_layout(kb, vb, n, false);
+  const bool wide = workspace_bytes < L.total;
+  if (wide) L = radix_layout(kb, vb, n, true);
   if (workspace_bytes < L.total) return hipErrorInvalidValue;
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   if (kb == 4) {
     uint32_t* k = reinterpret_cast<uint32_t*>(keys);
-    if (vb == 0) return radix_sort_s<uint32_t, 0>(k, vals, n, xf, ws, L, stream, timer, policy);
-    if (vb == 4) return radix_sort_s<uint32_t, 4>(k, vals, n, xf, ws, L, stream, timer, policy);
-    if (vb == 8) return radix_sort_s<uint32_t, 8>(k, vals, n, xf, ws, L, stream, timer, policy);
+    if (vb == 0) return radix_sort_v<uint32_t, 0>(k, vals, n, xf, ws, L, wide, stream, timer, policy);
+    if (vb == 4) return radix_sort_v<uint32_t, 4>(k, vals, n, xf, ws, L, wide, stream, timer, policy);
+    if (vb == 8) return radix_sort_v<uint32_t, 8>(k, vals, n, xf, ws, L, wide, stream, timer, policy);
   } else if (kb == 8) {
     uint64_t* k = reinterpret_cast<uint64_t*>(keys);
-    if (vb == 0) return radix_sort_s<uint64_t, 0>(k, vals, n, xf, ws, L, stream, timer, policy);
-    if (vb == 4) return radix_sort_s<uint64_t, 4>(k, vals, n, xf, ws, L, stream, timer, policy);
-    if (vb == 8) return radix_sort_s<uint64_t, 8>(k, vals, n, xf, ws, L, stream, timer, policy);
+    if (vb == 0) return radix_sort_v<uint64_t, 0>(k, vals, n, xf, ws, L, wide, stream, timer, policy);
+    if (vb == 4) return radix_sort_v<uint64_t, 4>(k, vals, n, xf, ws, L, wide, stream, timer, policy);
+    if (vb == 8) return radix_sort_v<uint64_t, 8>(k, vals, n, xf, ws, L, wide, stream, timer, policy);
   }
   return hipErrorInvalidValue;
 }

@@ -107,8 +107,8 @@ __device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint6
   return 0;
 }
 
-// Where the keys are: one array of n keys (tile_seg null) in the buffer that
-// ctrl->final_sel names, or the segments of a segmented sort, in buffer 0.
+// Where the keys are: one array of n keys (tile_seg null) or the segments of a
+// segmented sort, in buffer 0.
 template <typename V>
 struct TieArgs {
   uint64_t* keys0;
@@ -212,10 +212,6 @@ __global__ __launch_bounds__(256) void tie_fix_kernel(TieArgs<V> a) {
     start = seg0 + (uint64_t)(blockIdx.x - a.seg_first[slot]) * a.tile_keys;
   } else {
     start = (uint64_t)blockIdx.x * a.tile_keys;
-    if (a.ctrl->final_sel) {
-      keys = a.keys1;
-      vals = a.vals1;
-    }
   }
   end = start + a.tile_keys < seg1 ? start + a.tile_keys : seg1;
   for (uint64_t c0 = start; c0 < end; c0 += kTieChunk) {
@@ -328,11 +324,10 @@ __global__ __launch_bounds__(1024) void long_run_kernel(TieArgs<V> a) {
   const uint32_t count = a.ctrl->long_count, low = a.ctrl->low();
   const uint32_t tid = threadIdx.x;
   const int s = 8 * (int)low;
-  const bool alt = !a.tile_seg && a.ctrl->final_sel;
-  uint64_t* const keys = alt ? a.keys1 : a.keys0;
-  uint64_t* const other = alt ? a.keys0 : a.keys1;
-  V* const vals = alt ? a.vals1 : a.vals0;
-  V* const vother = alt ? a.vals0 : a.vals1;
+  uint64_t* const keys = a.keys0;
+  uint64_t* const other = a.keys1;
+  V* const vals = a.vals0;
+  V* const vother = a.vals1;
   for (uint32_t job = blockIdx.x; job < count; job += gridDim.x) {
     const uint64_t p0 = a.long_start[job];
     if (tid == 0) {
