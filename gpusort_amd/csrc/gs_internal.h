@@ -89,7 +89,7 @@ hipError_t radix_sort(int key_bytes, int val_bytes, void* keys, void* vals, uint
 // ping-pong buffer in the workspace mirrors the whole array); n_keys is the
 // number of keys in the segments.
 struct SegTiles {
-  int geo;  // tile geometry (radix_seg_tile_keys): 0 = the large one, 1-3 = the small-tile class's
+  int geo;  // tile geometry (radix_seg_tile_keys): 0, 4 = the large ones, 1-3 = the small-tile class's
   const uint32_t* tile_seg;
   const uint32_t* seg_first;
   const uint64_t* seg_range;
@@ -110,8 +110,11 @@ hipError_t multisplit(int key_bytes, int val_bytes, const void* keys, const void
                       void* out_vals, uint64_t* d_bucket_base, void* workspace, size_t workspace_bytes,
                       hipStream_t stream, LaunchTimer* timer = nullptr, int tile_policy = kTilesByStream);
 
-// Keys per tile of segmented-sort geometry `geo` (0 or 1).
+// Keys per tile of segmented-sort geometry `geo` (0-4).
 uint32_t radix_seg_tile_keys(int key_bytes, int val_bytes, int geo);
+// Geometry of the large class: 0, or 4 (smaller tiles) where that is better for
+// segments cut into `tiles` tiles of geometry 0 and tiles4 of geometry 4.
+int radix_seg_large_geo(int key_bytes, int val_bytes, uint64_t tiles, uint64_t tiles4);
 
 // Size classes of the batched segmented sort: segments of at most small_max
 // keys (<= block_sort_max) are sorted in LDS, those of at

@@ -1075,8 +1075,30 @@ struct SegGeometry<U, VB, 3> {
   static constexpr int THREADS = 512, ITEMS = SegGeometry<U, VB, 1>::ITEMS;
 };
 
+// Smaller large-class tiles for batches that are a round or two of tiles
+// (radix_seg_large_geo): 32-bit keys alone and with 32-bit payloads.
+template <>
+struct SegGeometry<uint32_t, 0, 4> {
+  static constexpr int THREADS = 1024, ITEMS = 18;
+};
+template <>
+struct SegGeometry<uint32_t, 4, 4> {
+  static constexpr int THREADS = 1024, ITEMS = 13;
+};
+
+// The large class's geometry for segments of which it makes `tiles` tiles, and
+// geometry 4 tiles4: the smaller tiles where they need no more rounds of a
+// tile a CU (as in sort_tile_of).
+int radix_seg_large_geo(int kb, int vb, uint64_t tiles, uint64_t tiles4) {
+  auto rounds = [](uint64_t t) { return (t + kRoundTiles - 1) / kRoundTiles; };
+  return kb == 4 && vb <= 4 && rounds(tiles) <= 2 && rounds(tiles4) == rounds(tiles) ? 4 : 0;
+}
+
 uint32_t radix_seg_tile_keys(int kb, int vb, int geo) {
-  if (geo == 0) {
+  if (geo == 4 && kb == 4 && vb <= 4)
+    return vb == 0 ? SegGeometry<uint32_t, 0, 4>::THREADS * SegGeometry<uint32_t, 0, 4>::ITEMS
+                   : SegGeometry<uint32_t, 4, 4>::THREADS * SegGeometry<uint32_t, 4, 4>::ITEMS;
+  if (geo == 0 || geo == 4) {
     if (kb == 4 && vb == 0) return SegGeometry<uint32_t, 0, 0>::THREADS * SegGeometry<uint32_t, 0, 0>::ITEMS;
     return tile_keys_for(kb, vb);
   }
@@ -1345,12 +1367,12 @@ struct SegHistArgs {
 // (runs of equal keys) is added once per digit by one lane.
 constexpr uint32_t kSegHistCopies = 4;
 
-template <typename U, bool IDENT, int LOW>
+template <typename U, bool IDENT, int LOW, int THREADS>
 __device__ __forceinline__ void seg_hist_from(const SegHistArgs<U>& a, uint32_t* s_hist) {  // [digit][value][copy]
   constexpr int MAXP = sizeof(U);  // one 8-bit digit per key byte (passes == MAXP); those from LOW up are counted
   const uint32_t tid = threadIdx.x, tile = blockIdx.x;
   const uint32_t copy = tid & (kSegHistCopies - 1);
-  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * kRadix * kSegHistCopies; i += 256) s_hist[i] = 0;
+  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * kRadix * kSegHistCopies; i += THREADS) s_hist[i] = 0;
   const uint32_t slot = a.tile_seg[tile];
   const uint64_t start = a.seg_range[2 * slot] + (uint64_t)(tile - a.seg_first[slot]) * a.tile_keys;
   const uint64_t seg_end = a.seg_range[2 * slot + 1];
@@ -1379,17 +1401,17 @@ __device__ __forceinline__ void seg_hist_from(const SegHistArgs<U>& a, uint32_t*
   // Four keys per thread in flight: the loads are issued before any is
   // counted.
   uint64_t i = start + tid;
-  for (; i + 3 * 256 < end; i += 4 * 256) {
-    const U k0 = a.keys[i], k1 = a.keys[i + 256], k2 = a.keys[i + 512], k3 = a.keys[i + 768];
+  for (; i + 3 * THREADS < end; i += 4 * THREADS) {
+    const U k0 = a.keys[i], k1 = a.keys[i + THREADS], k2 = a.keys[i + 2 * THREADS], k3 = a.keys[i + 3 * THREADS];
     count(k0);
     count(k1);
     count(k2);
     count(k3);
   }
-  for (; i < end; i += 256) count(a.keys[i]);
+  for (; i < end; i += THREADS) count(a.keys[i]);
   __syncthreads();
   uint32_t* dst = a.seg_cnt + (uint64_t)slot * a.passes * kRadix + LOW * kRadix;
-  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * kRadix; i += 256) {
+  for (uint32_t i = tid; i < (uint32_t)(MAXP - LOW) * kRadix; i += THREADS) {
     uint32_t c = 0;
 #pragma unroll
     for (uint32_t j = 0; j < kSegHistCopies; ++j) c += s_hist[i * kSegHistCopies + j];
@@ -1401,17 +1423,20 @@ __device__ __forceinline__ void seg_hist_from(const SegHistArgs<U>& a, uint32_t*
   }
 }
 
-template <typename U, bool IDENT>
-__global__ __launch_bounds__(256) void seg_hist_kernel(SegHistArgs<U> a) {
+// A tile a workgroup, of 256 threads, or of 1024 where the tiles leave CUs
+// short of waves (147 tiles of 28,672 f32 keys: 23 -> 9 us).
+template <typename U, bool IDENT, int THREADS>
+__global__ __launch_bounds__(THREADS) void seg_hist_kernel(SegHistArgs<U> a) {
   __shared__ uint32_t s_hist[sizeof(U) * kRadix * kSegHistCopies];
   const uint32_t tid = threadIdx.x, tile = blockIdx.x;
-  for (int p = 0; p < a.passes; ++p) a.status[p * a.status_per_pass + (uint64_t)tile * kRadix + tid] = 0;
+  if (tid < kRadix)
+    for (int p = 0; p < a.passes; ++p) a.status[p * a.status_per_pass + (uint64_t)tile * kRadix + tid] = 0;
   if constexpr (sizeof(U) == 8) {
     const uint32_t low = a.ctrl->low();
-    if (low >= 4) return seg_hist_from<U, IDENT, 4>(a, s_hist);
-    if (low >= 2) return seg_hist_from<U, IDENT, 2>(a, s_hist);
+    if (low >= 4) return seg_hist_from<U, IDENT, 4, THREADS>(a, s_hist);
+    if (low >= 2) return seg_hist_from<U, IDENT, 2, THREADS>(a, s_hist);
   }
-  seg_hist_from<U, IDENT, 0>(a, s_hist);
+  seg_hist_from<U, IDENT, 0, THREADS>(a, s_hist);
 }
 
 // The lowest digit to sort by of the first kLowSlots multi-tile segments of
@@ -1526,10 +1551,16 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
   h.status_per_pass = status_per_pass;
   h.ctrl = ctrl;
   if (timer) timer->begin("seg_hist", T.n_keys * sizeof(U), stream);
-  if (ident)
-    hipLaunchKernelGGL((seg_hist_kernel<U, true>), dim3((uint32_t)T.tiles), dim3(256), 0, stream, h);
+  const bool wide = T.tiles <= 4 * kRoundTiles;
+  const dim3 hist_grid((uint32_t)T.tiles);
+  if (ident && wide)
+    hipLaunchKernelGGL((seg_hist_kernel<U, true, 1024>), hist_grid, dim3(1024), 0, stream, h);
+  else if (ident)
+    hipLaunchKernelGGL((seg_hist_kernel<U, true, 256>), hist_grid, dim3(256), 0, stream, h);
+  else if (wide)
+    hipLaunchKernelGGL((seg_hist_kernel<U, false, 1024>), hist_grid, dim3(1024), 0, stream, h);
   else
-    hipLaunchKernelGGL((seg_hist_kernel<U, false>), dim3((uint32_t)T.tiles), dim3(256), 0, stream, h);
+    hipLaunchKernelGGL((seg_hist_kernel<U, false, 256>), hist_grid, dim3(256), 0, stream, h);
   if (timer) timer->end(stream);
   hipLaunchKernelGGL(seg_scan_kernel, dim3(T.nslots), dim3(256), 0, stream, cnt, L.passes, ctrl);
   for (int p = 0; p < L.passes; ++p) {
@@ -1594,6 +1625,11 @@ static hipError_t radix_segments_i(U* keys, void* vals, const SegTiles& T, const
   if (T.geo == 3)
     return small_idx ? radix_segments_t<U, VB, uint32_t, 3>(keys, vals, T, xp, ws, L, stream, timer, policy)
                      : radix_segments_t<U, VB, uint64_t, 3>(keys, vals, T, xp, ws, L, stream, timer, policy);
+  if constexpr (sizeof(U) == 4 && VB <= 4) {
+    if (T.geo == 4)
+      return small_idx ? radix_segments_t<U, VB, uint32_t, 4>(keys, vals, T, xp, ws, L, stream, timer, policy)
+                       : radix_segments_t<U, VB, uint64_t, 4>(keys, vals, T, xp, ws, L, stream, timer, policy);
+  }
   if (T.geo != 0) return hipErrorInvalidValue;
   if (T.n_total < (1ull << 32)) return radix_segments_t<U, VB, uint32_t, 0>(keys, vals, T, xp, ws, L, stream, timer, policy);
   return radix_segments_t<U, VB, uint64_t, 0>(keys, vals, T, xp, ws, L, stream, timer, policy);

@@ -121,6 +121,24 @@ void build_seg_plan(int kb, int vb, const uint64_t* off, uint32_t nseg, const Se
     next[l] = lists[l]->data();
   }
   for (uint32_t s = 0; s < nseg; ++s) *next[to[s]]++ = s;
+  // The large class takes smaller tiles where those need no more rounds of CUs.
+  {
+    std::vector<uint32_t> ids(P->multi_ids[0].size() + P->single_ids[0].size());
+    std::merge(P->multi_ids[0].begin(), P->multi_ids[0].end(), P->single_ids[0].begin(), P->single_ids[0].end(),
+               ids.begin());
+    uint64_t tiles[2] = {};
+    for (int i = 0; i < 2; ++i) {
+      const uint64_t t = radix_seg_tile_keys(kb, vb, 4 * i);
+      for (uint32_t s : ids) tiles[i] += (off[s + 1] - off[s] + t - 1) / t;
+    }
+    P->grp[0].geo = radix_seg_large_geo(kb, vb, tiles[0], tiles[1]);
+    if (P->grp[0].geo != 0) {
+      const uint64_t t = radix_seg_tile_keys(kb, vb, P->grp[0].geo);
+      P->multi_ids[0].clear();
+      P->single_ids[0].clear();
+      for (uint32_t s : ids) (off[s + 1] - off[s] > t ? P->multi_ids[0] : P->single_ids[0]).push_back(s);
+    }
+  }
   // Classes that together leave CUs idle share the launch of the longer one: a
   // launch lasts as long as its longest segment (4 us for the shortest class,
   // 40 for the longest), and launches follow one another.
