@@ -18,8 +18,8 @@
 //
 // What bounds it: the pull, at about 1 ms for 2^27 elements the rate of L2
 // accesses (one an element); then split and place, bytes (14 and, with u32, 10
-// an element).  Measured, 2^27 random indexes: u16 2.58 -> 1.54 ms, u32 2.56 ->
-// 1.71, u64 3.27 -> 2.28; 2^24: u32 0.314 -> 0.210, u64 0.337 -> 0.279.
+// an element).  Measured, 2^27 random indexes: u16 2.58 -> 1.31 ms, u32 2.56 ->
+// 1.53, u64 3.27 -> 2.09; 2^24: u32 0.314 -> 0.205, u64 0.337 -> 0.269.
 // In-order indexes cost the leaving kernels' 10-20 us (2^24 u32: 39 -> 50 us,
 // 2^27: 402 -> 422); below 2^24 elements that weighs more than the saving
 // (2^23 u32: 144 -> 108, u8 88 -> 96), so kGatherSplitMin lies there.
@@ -70,7 +70,7 @@ __device__ inline uint32_t slot_shift(uint32_t tile, uint32_t valid) {
 static_assert(kTile == 1u << 14, "slot_shift gives 14 bits");
 
 // What bounds it: the read of the indexes and the writes (14 bytes an element;
-// 2^27 of them 0.42 ms, 4.5 TB/s), two workgroups a CU overlapping their phases.
+// 2^27 of them 0.36 ms, 5.2 TB/s), two workgroups a CU overlapping their phases.
 __global__ __launch_bounds__(kThreads, 8) void gather_split_kernel(const uint64_t* __restrict__ idx, uint64_t n,
                                                                    uint32_t elem_bytes, uint32_t shift,
                                                                    uint32_t regions, uint32_t* __restrict__ split,
@@ -99,8 +99,8 @@ __global__ __launch_bounds__(kThreads, 8) void gather_split_kernel(const uint64_
   uint32_t wide = 0;
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
-    const uint32_t p = full ? (uint32_t)j * kThreads + tid : min((uint32_t)j * kThreads + tid, valid - 1);
-    const uint64_t v = ti[p];
+    const uint64_t v =
+        full ? (ti + j * (int)kThreads)[tid] : ti[min((uint32_t)j * kThreads + tid, valid - 1)];
     wide |= (uint32_t)(v >> 32);
     x[j] = (uint32_t)v;
   }
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kThreads, 8) void gather_split_kernel(const uint64_
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     const uint32_t p = (uint32_t)j * kThreads + tid;
-    if (full || p < valid) ent[base + p] = s_buf[p];
+    if (full || p < valid) (ent + base + j * (int)kThreads)[tid] = s_buf[p];
   }
   lds_barrier();
   uint16_t* const s_place = reinterpret_cast<uint16_t*>(s_buf);
@@ -233,8 +233,11 @@ __global__ __launch_bounds__(kPullThreads) void gather_pull_kernel(const T* __re
   }
 }
 
+// Two workgroups a CU but for 8-byte elements: at most 64 registers, which the
+// addresses stay within where the items' offsets are uniform (89 registers, one
+// workgroup: 0.39 ms for 2^27 u32 elements; 64: 0.25).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void gather_place_kernel(const T* __restrict__ src, const uint64_t* idx,
+__global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 4 : 8) void gather_place_kernel(const T* __restrict__ src, const uint64_t* idx,
                                                                 T* dst, uint64_t n, uint32_t regions,
                                                                 const uint32_t* __restrict__ split,
                                                                 const uint16_t* __restrict__ place,
@@ -247,28 +250,36 @@ __global__ __launch_bounds__(kThreads) void gather_place_kernel(const T* __restr
     T* const td = dst + (uint64_t)tile * kTile;
     if (valid == 0) {  // an index of 2^32 or more: not split
       const uint64_t base = (uint64_t)tile * kTile;
+#pragma unroll 1
       for (uint64_t p = base + tid; p < n && p < base + kTile; p += kThreads) dst[p] = src[idx[p]];
       continue;
     }
     const uint16_t* const tp = place + (uint64_t)tile * kTile;
     uint16_t at[kItems];
     T v[kItems];
+    if (valid == kTile) {
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const uint32_t p = (uint32_t)j * kThreads + tid;
-      if (p < valid) {
+      for (int j = 0; j < kItems; ++j) {
+        at[j] = (tp + j * (int)kThreads)[tid];
+        v[j] = (td + j * (int)kThreads)[tid];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < kItems; ++j) {
+        const uint32_t p = min((uint32_t)j * kThreads + tid, valid - 1);
         at[j] = tp[p];
         v[j] = td[p];
       }
     }
+    // Past the end of the last tile: its last element once more.
 #pragma unroll
-    for (int j = 0; j < kItems; ++j)
-      if ((uint32_t)j * kThreads + tid < valid) s_val[at[j]] = v[j];
+    for (int j = 0; j < kItems; ++j) s_val[at[j]] = v[j];
     lds_barrier();
+    if (valid == kTile) {
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const uint32_t p = (uint32_t)j * kThreads + tid;
-      if (p < valid) td[p] = s_val[p];
+      for (int j = 0; j < kItems; ++j) (td + j * (int)kThreads)[tid] = s_val[(uint32_t)j * kThreads + tid];
+    } else {
+      for (uint32_t p = tid; p < valid; p += kThreads) td[p] = s_val[p];
     }
     lds_barrier();
   }
