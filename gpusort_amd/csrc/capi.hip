@@ -202,7 +202,7 @@ hipError_t gather_device(gs_handle* h, int elem_bytes, const void* src, const ui
   hipError_t e = hipSuccess;
   if (h->gather_done == nullptr)
     e = hipEventCreateWithFlags(&h->gather_done, hipEventDisableTiming);
-  else if (h->stream != h->gather_stream)
+  else if (h->stream != h->gather_stream || h->stream != nullptr)  // a stream made anew may have an old one's address
     e = hipStreamWaitEvent(h->stream, h->gather_done, 0);
   if (e == hipSuccess) e = h->arena.get(Arena::kGather, bytes, h->stream, &ws);
   (void)hipThreadExchangeStreamCaptureMode(&mode);
