@@ -95,7 +95,6 @@ void Arena::release() {
 
 // ---------------------------------------------------------------- stage
 void* PinnedStage::take(size_t bytes, hipStream_t stream) {
-  bytes = align_up(bytes ? bytes : 1, 256);
   if (bytes > kBytes || failed_) return nullptr;
   if (!base_) {
     void* p = nullptr;
@@ -106,18 +105,14 @@ void* PinnedStage::take(size_t bytes, hipStream_t stream) {
     }
     base_ = static_cast<char*>(p);
   }
-  if (used_ + bytes > kBytes) {
-    if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
-    used_ = 0;
-  }
-  used_ += bytes;
-  return base_ + used_ - bytes;
+  const size_t at = ring_.take(bytes, [&] { return hipStreamSynchronize(stream) == hipSuccess; });
+  return at == StageRing::kNone ? nullptr : base_ + at;
 }
 
 void PinnedStage::release() {
   if (base_) (void)hipHostFree(base_);
   base_ = nullptr;
-  used_ = 0;
+  ring_.restart();
 }
 
 // ---------------------------------------------------------------- profiler

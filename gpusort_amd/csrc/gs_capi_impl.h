@@ -13,6 +13,7 @@
 
 #include "../../include/gpusort_hip.h"
 #include "gs_internal.h"
+#include "pinned_stage.h"
 
 namespace gs {
 
@@ -76,13 +77,14 @@ class PinnedStage {
  public:
   static constexpr size_t kBytes = 4u << 20;
   // Room for `bytes`, or null (too large, or no pinned memory): the caller then
-  // copies from and to its own memory.
+  // copies from and to its own memory.  Good until the next call may start over:
+  // blocks that are read together take one room (read_staged).
   void* take(size_t bytes, hipStream_t stream);
   void release();
 
  private:
   char* base_ = nullptr;
-  size_t used_ = 0;
+  StageRing ring_{kBytes};
   bool failed_ = false;
 };
 

@@ -66,25 +66,14 @@ struct Pipe {
 };
 
 // Copies blocks of device memory to host memory, and waits for them.
-struct ReadBlock {
-  void* dst;
-  const void* src;
-  size_t bytes;
-};
-
 hipError_t read_blocks(Pipe& P, std::initializer_list<ReadBlock> blocks) {
-  std::vector<std::pair<const ReadBlock*, void*>> staged;
-  for (const ReadBlock& b : blocks) {
-    if (b.bytes == 0) continue;
-    void* at = P.h->stage.take(b.bytes, P.h->stream);
-    if (at) staged.push_back({&b, at});
-    const hipError_t e = hipMemcpyAsync(at ? at : b.dst, b.src, b.bytes, hipMemcpyDeviceToHost, P.h->stream);
-    if (e != hipSuccess) return e;
-  }
-  const hipError_t e = hipStreamSynchronize(P.h->stream);
-  if (e != hipSuccess) return e;
-  for (const auto& s : staged) memcpy(s.first->dst, s.second, s.first->bytes);
-  return hipSuccess;
+  const hipStream_t stream = P.h->stream;
+  return read_staged(
+      blocks, [&](size_t bytes) { return P.h->stage.take(bytes, stream); },
+      [&](void* dst, const void* src, size_t bytes) {
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+      },
+      [&] { return hipStreamSynchronize(stream); });
 }
 
 bool is_pow2(uint64_t x) { return x && !(x & (x - 1)); }
