@@ -148,3 +148,18 @@ struct gs_handle {
     return it == seg_tuned.end() ? gs::default_seg_config(kb, vb) : it->second;
   }
 };
+
+namespace gs {
+
+// Waits for the handle's stream on every way out of a call but the one that has
+// waited already (done): what the call queued reads the pinned stage and vectors
+// of its frame.  Declared after them.
+struct DrainGuard {
+  gs_handle* h;
+  bool done = false;
+  ~DrainGuard() {
+    if (!done) (void)hipStreamSynchronize(h->stream);
+  }
+};
+
+}  // namespace gs

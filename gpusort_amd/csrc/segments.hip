@@ -282,6 +282,9 @@ extern "C" gs_status gs_sort_segments(gs_handle* h, gs_dtype kdt, void* d_keys, 
   std::vector<uint64_t>& off = h->seg_offsets;
   const size_t off_bytes = ((size_t)nseg + 1) * sizeof(uint64_t);
   off.resize((size_t)nseg + 1);
+  std::vector<unsigned char> meta;
+  std::vector<uint32_t> huge;
+  DrainGuard drain{h};
   void* const staged = h->stage.take(off_bytes, h->stream);
   hipError_t e = hipMemcpyAsync(staged ? staged : off.data(), d_offsets, off_bytes, hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
@@ -291,8 +294,6 @@ extern "C" gs_status gs_sort_segments(gs_handle* h, gs_dtype kdt, void* d_keys, 
     if (off[s + 1] < off[s]) return fail(GS_INVALID_ARG, "segment offsets decrease at segment %u", s);
   if (off[nseg] == off[0]) return GS_OK;  // every segment empty: nothing is read (null pointers allowed)
   if (!d_keys || (vdt != GS_NONE && !d_vals)) return fail(GS_INVALID_ARG, "null pointer");
-  std::vector<unsigned char> meta;
-  std::vector<uint32_t> huge;
   gs_status st = sort_segments_async(h, kdt, d_keys, vdt, d_vals, off.data(), nseg, descending, &meta, &huge);
   if (st != GS_OK) return st;
   char* kbase = reinterpret_cast<char*>(d_keys);
@@ -303,6 +304,7 @@ extern "C" gs_status gs_sort_segments(gs_handle* h, gs_dtype kdt, void* d_keys, 
     if (st != GS_OK) return st;
   }
   // The maps were copied from host memory owned by this frame.
+  drain.done = true;
   return from_hip(hipStreamSynchronize(h->stream), "segmented sort");
 }
 

@@ -777,6 +777,7 @@ extern "C" gs_status gs_vrank_sort(gs_handle* h, gs_algorithm algo, gs_dtype kdt
 
   DeviceScope ds(h->device);
   Pipe P;
+  DrainGuard drain{h};
   P.h = h;
   P.kdt = kdt;
   P.vdt = vdt;
@@ -855,6 +856,7 @@ extern "C" gs_status gs_vrank_sort(gs_handle* h, gs_algorithm algo, gs_dtype kdt
     if (e != hipSuccess) return from_hip(e, "copy result");
   }
   e = hipStreamSynchronize(h->stream);
+  drain.done = true;
   if (e != hipSuccess) return from_hip(e, "pipeline");
   if (report) {
     report->rounds = rounds;

@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from gpu_util import assert_bits_equal, dev, host, say
-from gpusort_amd import HYPERQUICKSORT, SAMPLESORT
+from gpusort_amd import HYKSORT, HYPERQUICKSORT, SAMPLESORT, GpusortError
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +42,29 @@ def test_samples_that_fill_the_buffer(handle, case):
         assert np.array_equal(got["final_rank_sizes"].astype(np.int64), want["final_rank_sizes"])
         assert_bits_equal(host(tk), want_k, "keys")
         assert_bits_equal(host(tv), want_v, "payloads")
+
+
+def test_a_call_that_fails_has_waited_for_its_stream(handle):
+    """An error in the middle of a rank sort (more samples than the selection
+    takes) leaves nothing queued that still reads the buffer."""
+    torch = pytest.importorskip("torch")
+    off = np.array([0, 30_000, 60_000], dtype=np.uint64)
+    keys = np.random.RandomState(3).randint(0, 1 << 31, 60_000).astype(np.uint32)
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+    tk = dev(keys)
+    torch.cuda.synchronize()
+    try:
+        handle.set_stream(stream)
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(20_000_000)
+        say("rank sort with too many samples")
+        with pytest.raises(GpusortError, match="exceeds"):
+            handle.vrank_sort(tk, off, algorithm=HYKSORT, k_way=2, samples_per_rank=1 << 24)
+        assert stream.query(), "the failed call left work queued"
+        handle.set_stream(other)
+        tk = dev(keys)
+        torch.cuda.synchronize()
+        handle.vrank_sort(tk, off, algorithm=HYKSORT, k_way=2, samples_per_rank=32)
+    finally:
+        handle.set_stream(0)
+    assert_bits_equal(host(tk), np.sort(keys), "keys")
