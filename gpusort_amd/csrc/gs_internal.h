@@ -36,18 +36,24 @@ constexpr uint32_t kCopyPass = 4;  // a pass that only copies from buffer (src &
 struct SortCtrl {
   uint32_t src[kMaxPasses];
   uint32_t tile_counter[kMaxPasses];
-  uint32_t unused[2];
+  uint32_t pad[16];
   // Tile tickets per workgroup class (blockIdx % 8) when a pass hands out
   // tiles in XCD groups.
   uint32_t class_counter[kMaxPasses][8];
-  uint32_t pad[14];
   // 64-bit keys (radix_ties.h): the number of highest digits sorted by (0:
-  // all), and the long runs listed for it.  In a cache line without ticket
-  // counters: every workgroup of a segmented pass reads it.
+  // all), and what is left to sort after them: the long runs listed, and of
+  // those that workgroups share the tasks handed out and done, the runs (high
+  // half) and their chunks (low half), and the bits that vary within one.  In a
+  // cache line without ticket counters of the passes: every workgroup of a
+  // segmented pass reads it.
   uint32_t top_digits;
   uint32_t long_count;
+  uint32_t task_counter;
+  uint32_t pad2;
+  unsigned long long shared;
+  unsigned long long shared_diff;
+  uint32_t done[24];
   __host__ __device__ uint32_t low() const { return top_digits ? 8u - top_digits : 0u; }
-  uint32_t pad2[30];
 };
 static_assert(sizeof(SortCtrl) == 512, "tickets in the first three 128-byte lines, top_digits in the fourth");
 

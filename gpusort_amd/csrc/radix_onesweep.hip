@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void radix_prep_kernel(uint32_t* __restrict__ 
                                                          const uint64_t* __restrict__ keys, uint64_t n,
                                                          Xform<uint64_t> xf) {
   __shared__ LowTile::Smem s_tile;
-  __shared__ uint32_t s_sum[8];
+  __shared__ uint32_t s_sum[16];
   const uint32_t tid = threadIdx.x;
   for (uint32_t i = blockIdx.x * 256 + tid; i < words; i += gridDim.x * 256) g_hist[i] = 0;
   if (blockIdx.x != 0) return;
@@ -259,10 +259,7 @@ __global__ __launch_bounds__(256) void radix_prep_kernel(uint32_t* __restrict__ 
       k[i] = to_ordered(keys[sample_pos((tid >> 6) * 256 + (uint32_t)i * 64 + (tid & 63u), n)], xf);
     low = choose_low(s_tile, k, n, false, s_sum);
   }
-  if (tid == 0) {
-    ctrl->top_digits = low ? 8 - low : 0;
-    ctrl->long_count = 0;
-  }
+  if (tid < kTieWords) (&ctrl->top_digits)[tid] = tid == 0 && low ? 8 - low : 0;
 }
 
 // Digit starts of every pass (a wave per digit position), and which passes
@@ -1281,10 +1278,10 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
     t.n = n;
     t.xf = xf;
     t.ctrl = ctrl;
-    t.use_status(status, status_per_pass * sizeof(S), L.tiles, THREADS * ITEMS);
+    t.template use_status<THREADS * ITEMS, KV>(status, L.tiles);
     // One chunk a workgroup up to 2^23 keys (four a CU at 2^21), then four.
     t.tile_keys = n <= (1ull << 23) ? kTieChunk : 4 * kTieChunk;
-    launch_tie_fix<V, KV>(t, (n + t.tile_keys - 1) / t.tile_keys, n, stream, timer);
+    launch_tie_fix<V, KV, S>(t, (n + t.tile_keys - 1) / t.tile_keys, n, stream, timer);
   }
   return hipGetLastError();
 }
@@ -1439,18 +1436,18 @@ __global__ __launch_bounds__(THREADS) void seg_hist_kernel(SegHistArgs<U> a) {
   seg_hist_from<U, IDENT, 0, THREADS>(a, s_hist);
 }
 
-// The lowest digit to sort by of the first kLowSlots multi-tile segments of
-// 64-bit keys, a workgroup each (four or six digits, so that the result lands
-// where the keys were): the largest number of digits counts.
-constexpr uint32_t kLowSlots = 2048;
-
+// The lowest digit to sort by of segments of 64-bit keys, a workgroup each (four
+// or six digits, so that the result lands where the keys were): the largest
+// number of digits counts.  A segment of fewer keys than four samples has no
+// say: all of it fits one workgroup's tile if its keys agree above.
 __global__ __launch_bounds__(256) void seg_prep_kernel(SortCtrl* ctrl, const uint64_t* __restrict__ keys,
                                                        const uint64_t* __restrict__ seg_range, Xform<uint64_t> xf) {
   __shared__ LowTile::Smem s_tile;
-  __shared__ uint32_t s_sum[8];
+  __shared__ uint32_t s_sum[16];
   const uint32_t tid = threadIdx.x;
   const uint64_t start = seg_range[2 * blockIdx.x];
   const uint64_t len = seg_range[2 * blockIdx.x + 1] - start;
+  if (len < 4 * kLowSample) return;
   uint64_t k[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -1531,11 +1528,11 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
   hipError_t e = fill_u32(reinterpret_cast<uint32_t*>(ws + L.off_ctrl),
                           (L.off_cnt - L.off_ctrl) / 4 + (uint64_t)T.n_multi * L.passes * kRadix, 0u, stream);
   if (e != hipSuccess) return e;
-  // Every multi-tile segment holds more than a sample's keys.
-  const uint32_t sampled = sizeof(U) == 8 ? std::min(T.n_multi, kLowSlots) : 0;
+  // Batches of nothing but single-tile segments sort by every digit.
+  const bool by_top = sizeof(U) == 8 && T.n_multi != 0;
   if constexpr (sizeof(U) == 8) {
-    if (sampled)
-      hipLaunchKernelGGL(seg_prep_kernel, dim3(sampled), dim3(256), 0, stream, ctrl, (const U*)keys, T.seg_range, xf);
+    if (by_top)
+      hipLaunchKernelGGL(seg_prep_kernel, dim3(T.nslots), dim3(256), 0, stream, ctrl, (const U*)keys, T.seg_range, xf);
   }
   SegHistArgs<U> h;
   h.keys = keys;
@@ -1593,7 +1590,7 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
     if (timer) timer->end(stream);
   }
   if constexpr (sizeof(U) == 8) {
-    if (sampled) {
+    if (by_top) {
       TieArgs<V> t{};
       t.keys0 = keys;
       t.keys1 = reinterpret_cast<U*>(ws + L.off_keys_tmp);
@@ -1605,8 +1602,8 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
       t.tile_seg = T.tile_seg;
       t.seg_first = T.seg_first;
       t.seg_range = T.seg_range;
-      t.use_status(status, status_per_pass * sizeof(uint32_t), T.tiles, THREADS * ITEMS);
-      launch_tie_fix<V, KV>(t, T.tiles, T.n_keys, stream, timer);
+      t.template use_status<THREADS * ITEMS, KV>(status, T.tiles);
+      launch_tie_fix<V, KV, uint32_t>(t, T.tiles, T.n_keys, stream, timer);
     }
   }
   return hipGetLastError();
