@@ -12,8 +12,8 @@
 //   place  every tile of dst put in order of place through LDS
 //
 // Nothing crosses a tile but the pull's reads of src, so there is no
-// histogram, scan or look-back.  Where neighbouring indexes are close together
-// already the three kernels leave and a fourth gathers directly; a tile that
+// histogram, scan or look-back.  Where the indexes are better gathered directly
+// (direct_is_better) the three kernels leave and a fourth gathers directly; a tile that
 // holds an index of 2^32 or more is gathered directly by the place kernel.
 //
 // What bounds it: the pull, at about 1 ms for 2^27 elements the rate of L2
@@ -47,10 +47,11 @@ constexpr uint64_t kRegionBytes = 2u << 20;
 // spread over the array: over a third of them are so close that they find each
 // other's lines in the L2, or all indexes lie in so little of src that caches
 // hold most of it (against the split, random indexes over 8 MB cost 10 ps an
-// element, over 32 MB 17; the split 12 and, with 8-byte elements, 18).  Every
-// wave of every workgroup finds the same answer.
+// element, over 32 MB 17; the split 12 and, with 8-byte elements, 18), or they
+// lie in so much of it that hardly two of them share a line: a quarter of them
+// are `far` or more.  Every wave of every workgroup finds the same answer.
 constexpr uint32_t kNearBytes = 256u << 10;
-__device__ inline bool direct_is_better(const uint64_t* idx, uint64_t n, uint32_t elem_bytes) {
+__device__ inline bool direct_is_better(const uint64_t* idx, uint64_t n, uint32_t elem_bytes, uint64_t far) {
   const uint32_t lane = threadIdx.x & 31u;
   const uint64_t a = idx[(n - 1) / 16 * (lane >> 1) + (lane & 1u)];
   const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)a, 0xB1, 0xf, 0xf, false);
@@ -58,7 +59,17 @@ __device__ inline bool direct_is_better(const uint64_t* idx, uint64_t n, uint32_
   const uint64_t b = ((uint64_t)hi << 32) | lo;
   const uint64_t small = (elem_bytes == 8 ? 48u << 20 : 14u << 20) / elem_bytes;
   return __popcll(ballot((a < b ? b - a : a - b) < kNearBytes / elem_bytes)) >= 24 ||  // a pair counts four times
-         ballot(a >= small) == 0;
+         ballot(a >= small) == 0 || __popcll(ballot(a >= far)) >= 16;                  // an index twice
+}
+
+// Three quarters of the elements of a source in which n random indexes fall on a
+// line of 128 bytes 0.8 times each, below 2^25 indexes 1.5 times: past that the
+// split costs more than it saves (2^24 indexes: u32 over 16 times as many elements
+// 364 us directly and 349 split, over 32 times 404 and 425; u64 over 4 times 339
+// and 337, over 16 times 432 and 466; 2^25: u64 over 16 times as many 948 and 911,
+// over 24 times 968 and 986).
+uint64_t far_index(uint64_t n, uint32_t elem_bytes) {
+  return n * (n < (1ull << 25) ? 64 : 120) / elem_bytes;
 }
 
 // Where a tile's slots start in its part of ent, place and dst.  Tiles are
@@ -72,7 +83,7 @@ static_assert(kTile == 1u << 14, "slot_shift gives 14 bits");
 // What bounds it: the read of the indexes and the writes (14 bytes an element;
 // 2^27 of them 0.36 ms, 5.2 TB/s), two workgroups a CU overlapping their phases.
 __global__ __launch_bounds__(kThreads, 8) void gather_split_kernel(const uint64_t* __restrict__ idx, uint64_t n,
-                                                                   uint32_t elem_bytes, uint32_t shift,
+                                                                   uint32_t elem_bytes, uint64_t far, uint32_t shift,
                                                                    uint32_t regions, uint32_t* __restrict__ split,
                                                                    uint32_t* __restrict__ tickets,
                                                                    uint32_t* __restrict__ ent,
@@ -81,7 +92,7 @@ __global__ __launch_bounds__(kThreads, 8) void gather_split_kernel(const uint64_
   __shared__ uint32_t s_cnt[kMaxRegions];
   __shared__ uint32_t s_buf[kTile];
   const uint32_t tid = threadIdx.x;
-  const bool direct = direct_is_better(idx, n, elem_bytes);
+  const bool direct = direct_is_better(idx, n, elem_bytes, far);
   if (blockIdx.x == 0) {
     if (tid == 0) *split = !direct;
     if (tid < kXcds) tickets[tid * 32] = 0;
@@ -327,7 +338,7 @@ hipError_t gather_split_t(const T* src, const uint64_t* idx, T* dst, uint64_t n,
   uint32_t shift = 0;
   while (((n - 1) >> shift) >= regions) ++shift;
   hipLaunchKernelGGL(gather_split_kernel, dim3(tiles), dim3(kThreads), 0, stream, idx, n,
-                     (uint32_t)sizeof(T), shift, regions, split, tickets, ent, place, rows);
+                     (uint32_t)sizeof(T), far_index(n, sizeof(T)), shift, regions, split, tickets, ent, place, rows);
   hipLaunchKernelGGL(gather_pull_kernel<T>, dim3(kXcds * kPullGroups), dim3(kPullThreads), 0, stream, src, dst, n,
                      regions, split, tickets, ent, rows);
   hipLaunchKernelGGL(gather_place_kernel<T>, dim3(std::min(tiles, 512u)), dim3(kThreads), 0, stream, src, idx, dst, n,

@@ -49,6 +49,52 @@ def test_gather_over_its_indexes(handle):
     assert torch.equal(idx, want)
 
 
+@pytest.mark.parametrize("width,times", [(1, 40), (2, 24), (4, 15), (4, 25), (8, 7), (8, 13)])
+def test_gather_from_a_sparse_source(handle, width, times):
+    """Sources far larger than the index vector, on both sides of where the split
+    gives way to a direct gather."""
+    n = N + 11
+    src, idx = _source(width, times * n), _indexes("random", n, times * n)
+    dst = torch.zeros(n, dtype=src.dtype, device="cuda")
+    say(f"gather from {times} times as many elements, width={width}")
+    handle.gather(src, idx, dst)
+    assert torch.equal(dst, src[idx])
+
+
+def _best_ms(call) -> float:
+    call()
+    ms = []
+    for _ in range(5):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        t0.record()
+        for _ in range(5):
+            call()
+        t1.record()
+        torch.cuda.synchronize()
+        ms.append(t0.elapsed_time(t1) / 5)
+    return min(ms)
+
+
+def test_gather_from_a_sparse_source_costs_no_more(handle):
+    """Where hardly two indexes share a line the call takes what a direct gather (a
+    captured call) does, not the split's passes on top (a quarter more)."""
+    src, idx = _source(8, 64 * N), _indexes("random", N, 64 * N)
+    dst = torch.zeros(N, dtype=torch.int64, device="cuda")
+    handle.gather(src, idx, dst)
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            handle.set_stream(torch.cuda.current_stream().cuda_stream)
+            handle.gather(src, idx, dst)
+    finally:
+        handle.set_stream(0)
+    say("time of a sparse gather")
+    direct, call = _best_ms(graph.replay), _best_ms(lambda: handle.gather(src, idx, dst))
+    print(direct, call)
+    assert call < 1.12 * direct
+
+
 def test_gather_on_changing_streams(handle):
     """Two streams in turn: the scratch of one call is not written by the next
     before it is read."""
