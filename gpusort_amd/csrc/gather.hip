@@ -13,16 +13,20 @@
 //
 // Nothing crosses a tile but the pull's reads of src, so there is no
 // histogram, scan or look-back.  Where the indexes are better gathered directly
-// (direct_is_better) the three kernels leave and a fourth gathers directly; a tile that
-// holds an index of 2^32 or more is gathered directly by the place kernel.
+// (direct_is_better) the split kernel leaves, the pull's workgroups gather and the
+// place kernel leaves.  An index of 2^32 or more is split as what it is below
+// that, an element of the source too, and gathered again by the place kernel;
+// where dst lies over idx such a tile is gathered directly, at the end.
 //
 // What bounds it: the pull, at about 1 ms for 2^27 elements the rate of L2
 // accesses (one an element); then split and place, bytes (14 and, with u32, 10
 // an element).  Measured, 2^27 random indexes: u16 2.58 -> 1.31 ms, u32 2.56 ->
 // 1.53, u64 3.27 -> 2.09; 2^24: u32 0.314 -> 0.205, u64 0.337 -> 0.269.
-// In-order indexes cost the leaving kernels' 10-20 us (2^24 u32: 39 -> 50 us,
-// 2^27: 402 -> 422); below 2^24 elements that weighs more than the saving
-// (2^23 u32: 144 -> 108, u8 88 -> 96), so kGatherSplitMin lies there.
+// In-order indexes cost the leaving kernels' 10 us (2^24 u32: 38 -> 48 us, 2^25
+// 97 -> 108); below 2^24 elements that weighs more than the saving (2^23 u32: 144
+// -> 108, u8 88 -> 96), so kGatherSplitMin lies there.  Gathering in the split
+// kernel instead leaves one kernel less, but its large workgroups lose the lines
+// that neighbours share (2^24 u32 shuffled within 64 K elements: 122 -> 176 us).
 #include <algorithm>
 
 #include "block_radix.h"
@@ -67,9 +71,9 @@ __device__ inline bool direct_is_better(const uint64_t* idx, uint64_t n, uint32_
 // split costs more than it saves (2^24 indexes: u32 over 16 times as many elements
 // 364 us directly and 349 split, over 32 times 404 and 425; u64 over 4 times 339
 // and 337, over 16 times 432 and 466; 2^25: u64 over 16 times as many 948 and 911,
-// over 24 times 968 and 986).
+// over 24 times 968 and 986).  At most 2^32, where a split index ends.
 uint64_t far_index(uint64_t n, uint32_t elem_bytes) {
-  return n * (n < (1ull << 25) ? 64 : 120) / elem_bytes;
+  return std::min<uint64_t>(n * (n < (1ull << 25) ? 64 : 120) / elem_bytes, 1ull << 32);
 }
 
 // Where a tile's slots start in its part of ent, place and dst.  Tiles are
@@ -82,99 +86,103 @@ static_assert(kTile == 1u << 14, "slot_shift gives 14 bits");
 
 // What bounds it: the read of the indexes and the writes (14 bytes an element;
 // 2^27 of them 0.36 ms, 5.2 TB/s), two workgroups a CU overlapping their phases.
+// `apart`: dst does not lie over idx.
 __global__ __launch_bounds__(kThreads, 8) void gather_split_kernel(const uint64_t* __restrict__ idx, uint64_t n,
-                                                                   uint32_t elem_bytes, uint64_t far, uint32_t shift,
-                                                                   uint32_t regions, uint32_t* __restrict__ split,
+                                                                   uint32_t elem_bytes, uint64_t far, bool apart,
+                                                                   uint32_t shift, uint32_t regions,
+                                                                   uint32_t* __restrict__ split,
                                                                    uint32_t* __restrict__ tickets,
                                                                    uint32_t* __restrict__ ent,
                                                                    uint16_t* __restrict__ place,
                                                                    uint16_t* __restrict__ rows) {
   __shared__ uint32_t s_cnt[kMaxRegions];
   __shared__ uint32_t s_buf[kTile];
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x, tile = blockIdx.x;
   const bool direct = direct_is_better(idx, n, elem_bytes, far);
-  if (blockIdx.x == 0) {
+  if (tile == 0) {
     if (tid == 0) *split = !direct;
     if (tid < kXcds) tickets[tid * 32] = 0;
   }
   if (direct) return;
-  const uint32_t tile = blockIdx.x;
   const uint64_t base = (uint64_t)tile * kTile;
   const uint32_t valid = n - base < kTile ? (uint32_t)(n - base) : kTile;
   // Compiled twice, for whole tiles (no compares) and for the last one.
   auto tile_body = [&](auto full_tag) {
-  constexpr bool full = decltype(full_tag)::value;
-  const uint64_t* const ti = idx + base;
-  for (uint32_t i = tid; i < kMaxRegions; i += kThreads) s_cnt[i] = 0;
-  uint32_t x[kItems];
-  uint32_t wide = 0;
+    constexpr bool full = decltype(full_tag)::value;
+    const uint64_t* const ti = idx + base;
+    for (uint32_t i = tid; i < kMaxRegions; i += kThreads) s_cnt[i] = 0;
+    uint32_t x[kItems];
+    uint32_t wide = 0;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint64_t v =
-        full ? (ti + j * (int)kThreads)[tid] : ti[min((uint32_t)j * kThreads + tid, valid - 1)];
-    wide |= (uint32_t)(v >> 32);
-    x[j] = (uint32_t)v;
-  }
-  uint16_t* const row = rows + (uint64_t)tile * kRow;
-  if (__syncthreads_or(wide != 0)) {
-    for (uint32_t i = tid; i < kRow; i += kThreads) row[i] = 0;
-    return;
-  }
-  const uint32_t skew = slot_shift(tile, valid);
-  auto region = [&](uint32_t v) { return (v >> shift) & (regions - 1); };
-  uint32_t r[kItems];
-#pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t p = (uint32_t)j * kThreads + tid;
-    r[j] = full || p < valid ? atomicAdd(&s_cnt[region(x[j])], 1u) : 0u;
-  }
-  lds_barrier();
-  if (tid < kWave) {  // one wave: starts of the regions
-    constexpr uint32_t PER = kMaxRegions / kWave / 4;
-    uint4* const c = reinterpret_cast<uint4*>(s_cnt) + PER * tid;
-    uint4 a[PER];
-    uint32_t sum = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < PER; ++i) {
-      a[i] = c[i];
-      sum += a[i].x + a[i].y + a[i].z + a[i].w;
+    for (int j = 0; j < kItems; ++j) {
+      const uint64_t v =
+          full ? (ti + j * (int)kThreads)[tid] : ti[min((uint32_t)j * kThreads + tid, valid - 1)];
+      wide |= (uint32_t)(v >> 32);
+      x[j] = (uint32_t)v;
     }
-    uint32_t at = wave_incl_scan_dpp(sum) - sum;
-#pragma unroll
-    for (uint32_t i = 0; i < PER; ++i) {
-      const uint4 y = make_uint4(at, at + a[i].x, at + a[i].x + a[i].y, at + a[i].x + a[i].y + a[i].z);
-      at = y.w + a[i].w;
-      c[i] = y;
+    uint16_t* const row = rows + (uint64_t)tile * kRow;
+    const bool any_wide = __syncthreads_or(wide != 0);
+    if (any_wide && !apart) {
+      for (uint32_t i = tid; i < kRow; i += kThreads) row[i] = 0;
+      return;
     }
-  }
-  lds_barrier();
-  for (uint32_t i = tid; i <= regions; i += kThreads) row[i] = (uint16_t)(i < regions ? s_cnt[i] : valid);
+    if (tid == 0) row[regions + 1] = any_wide;
+    const uint32_t skew = slot_shift(tile, valid);
+    auto region = [&](uint32_t v) { return (v >> shift) & (regions - 1); };
+    uint32_t r[kItems];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    r[j] = (r[j] + s_cnt[region(x[j])] + skew) % kTile;
-    if (full || (uint32_t)j * kThreads + tid < valid) s_buf[r[j]] = x[j];
-  }
-  lds_barrier();
+    for (int j = 0; j < kItems; ++j) {
+      const uint32_t p = (uint32_t)j * kThreads + tid;
+      r[j] = full || p < valid ? atomicAdd(&s_cnt[region(x[j])], 1u) : 0u;
+    }
+    lds_barrier();
+    if (tid < kWave) {  // one wave: starts of the regions
+      constexpr uint32_t PER = kMaxRegions / kWave / 4;
+      uint4* const c = reinterpret_cast<uint4*>(s_cnt) + PER * tid;
+      uint4 a[PER];
+      uint32_t sum = 0;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t p = (uint32_t)j * kThreads + tid;
-    if (full || p < valid) (ent + base + j * (int)kThreads)[tid] = s_buf[p];
-  }
-  lds_barrier();
-  uint16_t* const s_place = reinterpret_cast<uint16_t*>(s_buf);
+      for (uint32_t i = 0; i < PER; ++i) {
+        a[i] = c[i];
+        sum += a[i].x + a[i].y + a[i].z + a[i].w;
+      }
+      uint32_t at = wave_incl_scan_dpp(sum) - sum;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t p = (uint32_t)j * kThreads + tid;
-    if (full || p < valid) s_place[r[j]] = (uint16_t)p;
-  }
-  lds_barrier();
-  // The last tile's pairs past its end stay within the tile's part of place.
-  uint32_t* const pw = reinterpret_cast<uint32_t*>(place + base);
+      for (uint32_t i = 0; i < PER; ++i) {
+        const uint4 y = make_uint4(at, at + a[i].x, at + a[i].x + a[i].y, at + a[i].x + a[i].y + a[i].z);
+        at = y.w + a[i].w;
+        c[i] = y;
+      }
+    }
+    lds_barrier();
+    for (uint32_t i = tid; i <= regions; i += kThreads) row[i] = (uint16_t)(i < regions ? s_cnt[i] : valid);
 #pragma unroll
-  for (int j = 0; j < kItems / 2; ++j) {
-    const uint32_t p = (uint32_t)j * kThreads + tid;
-    if (full || 2 * p < valid) pw[p] = s_buf[p];
-  }  };
+    for (int j = 0; j < kItems; ++j) {
+      r[j] = (r[j] + s_cnt[region(x[j])] + skew) % kTile;
+      if (full || (uint32_t)j * kThreads + tid < valid) s_buf[r[j]] = x[j];
+    }
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const uint32_t p = (uint32_t)j * kThreads + tid;
+      if (full || p < valid) (ent + base + j * (int)kThreads)[tid] = s_buf[p];
+    }
+    lds_barrier();
+    uint16_t* const s_place = reinterpret_cast<uint16_t*>(s_buf);
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const uint32_t p = (uint32_t)j * kThreads + tid;
+      if (full || p < valid) s_place[r[j]] = (uint16_t)p;
+    }
+    lds_barrier();
+    // The last tile's pairs past its end stay within the tile's part of place.
+    uint32_t* const pw = reinterpret_cast<uint32_t*>(place + base);
+#pragma unroll
+    for (int j = 0; j < kItems / 2; ++j) {
+      const uint32_t p = (uint32_t)j * kThreads + tid;
+      if (full || 2 * p < valid) pw[p] = s_buf[p];
+    }
+  };
   if (valid == kTile)
     tile_body(std::true_type{});
   else
@@ -190,15 +198,24 @@ constexpr int kPullUnroll = 8;
 // ms, 4 a CU 1.74, 3 a CU 1.71, 2 a CU 1.75).  Dealing the jobs by ticket rather
 // than by stride keeps them to one region or two: 2.46 -> 1.91.
 constexpr uint32_t kPullGroups = 96;
+// Workgroups launched, all of which gather where the tiles were not split (one
+// launch less than with a kernel of its own).
+constexpr uint32_t kPullGrid = 8192;
 
 template <typename T>
-__global__ __launch_bounds__(kPullThreads) void gather_pull_kernel(const T* __restrict__ src, T* __restrict__ dst,
-                                                                   uint64_t n, uint32_t regions,
+__global__ __launch_bounds__(kPullThreads) void gather_pull_kernel(const T* __restrict__ src, const uint64_t* idx,
+                                                                   T* dst, uint64_t n, uint32_t regions,
                                                                    const uint32_t* __restrict__ split,
                                                                    uint32_t* __restrict__ tickets,
                                                                    const uint32_t* __restrict__ ent,
                                                                    const uint16_t* __restrict__ rows) {
-  if (!*split) return;
+  if (!*split) {
+    const uint64_t stride = (uint64_t)gridDim.x * kPullThreads;
+    for (uint64_t i = (uint64_t)blockIdx.x * kPullThreads + threadIdx.x; i < n; i += stride) dst[i] = src[idx[i]];
+    return;
+  }
+  constexpr uint32_t kWorkgroups = kXcds * kPullGroups;
+  if (blockIdx.x >= kWorkgroups) return;
   constexpr int UN = kPullUnroll;
   const uint32_t tiles = (uint32_t)((n + kTile - 1) / kTile);
   const uint32_t xcd = blockIdx.x % kXcds;
@@ -235,7 +252,7 @@ __global__ __launch_bounds__(kPullThreads) void gather_pull_kernel(const T* __re
   uint32_t job = blockIdx.x / kXcds;
   for (uint32_t turn = 0; job < jobs; turn ^= 1) {
     uint32_t next = 0;
-    if (threadIdx.x == 0) next = gridDim.x / kXcds + atomicAdd(&tickets[xcd * 32], 1u);
+    if (threadIdx.x == 0) next = kPullGroups + atomicAdd(&tickets[xcd * 32], 1u);
     const uint32_t b = xcd + kXcds * (job / chunks), tile = job % chunks * kPullTiles + group;
     if (tile < tiles) pull(b, tile);
     if (threadIdx.x == 0) s_job[turn] = next;
@@ -248,23 +265,23 @@ __global__ __launch_bounds__(kPullThreads) void gather_pull_kernel(const T* __re
 // addresses stay within where the items' offsets are uniform (89 registers, one
 // workgroup: 0.39 ms for 2^27 u32 elements; 64: 0.25).
 template <typename T>
-__global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 4 : 8) void gather_place_kernel(const T* __restrict__ src, const uint64_t* idx,
-                                                                T* dst, uint64_t n, uint32_t regions,
-                                                                const uint32_t* __restrict__ split,
-                                                                const uint16_t* __restrict__ place,
-                                                                const uint16_t* __restrict__ rows) {
+__global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 4 : 8) void gather_place_kernel(
+    const T* __restrict__ src, const uint64_t* idx, T* dst, uint64_t n, bool apart, uint32_t regions,
+    const uint32_t* __restrict__ split, const uint16_t* __restrict__ place, const uint16_t* __restrict__ rows) {
   __shared__ T s_val[kTile];
   if (!*split) return;
   const uint32_t tid = threadIdx.x, tiles = (uint32_t)((n + kTile - 1) / kTile);
   for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const uint32_t valid = rows[(uint64_t)tile * kRow + regions];
-    T* const td = dst + (uint64_t)tile * kTile;
-    if (valid == 0) {  // an index of 2^32 or more: not split
-      const uint64_t base = (uint64_t)tile * kTile;
-#pragma unroll 1
+    const uint64_t base = (uint64_t)tile * kTile;
+    T* const td = dst + base;
+    const uint16_t* const row = rows + (uint64_t)tile * kRow + regions;
+    const uint32_t valid = row[0];
+    if (valid == 0) {  // not split, dst lies over idx
+#pragma unroll 4
       for (uint64_t p = base + tid; p < n && p < base + kTile; p += kThreads) dst[p] = src[idx[p]];
       continue;
     }
+    const bool wide = row[1] != 0;
     const uint16_t* const tp = place + (uint64_t)tile * kTile;
     uint16_t at[kItems];
     T v[kItems];
@@ -293,16 +310,13 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 4 : 8) void gather_place
       for (uint32_t p = tid; p < valid; p += kThreads) td[p] = s_val[p];
     }
     lds_barrier();
+    if (wide)
+#pragma unroll 4
+      for (uint32_t p = tid; p < valid; p += kThreads) {
+        const uint64_t x = idx[base + p];
+        if (x >> 32) td[p] = src[x];
+      }
   }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void gather_direct_kernel(const T* __restrict__ src,
-                                                            const uint64_t* __restrict__ idx, T* __restrict__ dst,
-                                                            uint64_t n, const uint32_t* __restrict__ split) {
-  if (*split) return;
-  const uint64_t stride = (uint64_t)gridDim.x * 256;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) dst[i] = src[idx[i]];
 }
 
 struct GatherLayout {
@@ -337,13 +351,14 @@ hipError_t gather_split_t(const T* src, const uint64_t* idx, T* dst, uint64_t n,
   const uint32_t regions = n * sizeof(T) > kMinRegions * kRegionBytes ? kMaxRegions : kMinRegions;
   uint32_t shift = 0;
   while (((n - 1) >> shift) >= regions) ++shift;
-  hipLaunchKernelGGL(gather_split_kernel, dim3(tiles), dim3(kThreads), 0, stream, idx, n,
-                     (uint32_t)sizeof(T), far_index(n, sizeof(T)), shift, regions, split, tickets, ent, place, rows);
-  hipLaunchKernelGGL(gather_pull_kernel<T>, dim3(kXcds * kPullGroups), dim3(kPullThreads), 0, stream, src, dst, n,
-                     regions, split, tickets, ent, rows);
+  const uintptr_t di = reinterpret_cast<uintptr_t>(dst), ii = reinterpret_cast<uintptr_t>(idx);
+  const bool apart = di + n * sizeof(T) <= ii || ii + n * sizeof(uint64_t) <= di;
+  hipLaunchKernelGGL(gather_split_kernel, dim3(tiles), dim3(kThreads), 0, stream, idx, n, (uint32_t)sizeof(T),
+                     far_index(n, sizeof(T)), apart, shift, regions, split, tickets, ent, place, rows);
+  hipLaunchKernelGGL(gather_pull_kernel<T>, dim3(kPullGrid), dim3(kPullThreads), 0, stream, src, idx, dst, n, regions,
+                     split, tickets, ent, rows);
   hipLaunchKernelGGL(gather_place_kernel<T>, dim3(std::min(tiles, 512u)), dim3(kThreads), 0, stream, src, idx, dst, n,
-                     regions, split, place, rows);
-  hipLaunchKernelGGL(gather_direct_kernel<T>, dim3(8192), dim3(256), 0, stream, src, idx, dst, n, split);
+                     apart, regions, split, place, rows);
   return hipGetLastError();
 }
 

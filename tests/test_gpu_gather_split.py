@@ -95,6 +95,50 @@ def test_gather_from_a_sparse_source_costs_no_more(handle):
     assert call < 1.12 * direct
 
 
+@pytest.mark.parametrize("every", [1, 3, 100, N])
+def test_gather_of_indexes_past_32_bits(handle, every):
+    """One index in `every` lies past 2^32: such an element is gathered again after
+    its tile was put in place; most of them, and all is gathered directly."""
+    n = N + 5
+    src = torch.zeros((1 << 32) + n, dtype=torch.uint8, device="cuda")
+    src[:n] = _source(1, n)
+    src[1 << 32:] = _source(1, n) + 101
+    idx = _indexes("random", n, n)
+    idx[::every] += 1 << 32
+    dst = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    say(f"gather, one index in {every} past 2^32")
+    handle.gather(src, idx, dst)
+    assert torch.equal(dst, src[idx])
+
+
+def test_gather_over_its_indexes_past_32_bits(handle):
+    """dst over idx: a tile with such an index is left to the last kernel."""
+    n = N + 5
+    src = torch.empty((1 << 32) + n, dtype=torch.int64, device="cuda")
+    src[:n] = _source(8, n)
+    src[1 << 32:] = _source(8, n) * 3
+    idx = _indexes("random", n, n)
+    idx[::50_000] += 1 << 32
+    want = src[idx]
+    say("gather over its indexes, some past 2^32")
+    handle.gather(src, idx, idx)
+    assert torch.equal(idx, want)
+
+
+def test_few_indexes_past_32_bits_cost_no_multiple(handle):
+    """One index in a hundred past 2^32 leaves no tile of 16,384 without one: such a
+    gather took 2.2 times as long as one without."""
+    n = 2 * N
+    src = torch.zeros((1 << 32) + n, dtype=torch.uint8, device="cuda")
+    idx, dst = _indexes("random", n, n), torch.zeros(n, dtype=torch.uint8, device="cuda")
+    say("time of a gather with indexes past 2^32")
+    ms = [_best_ms(lambda: handle.gather(src, idx, dst))]
+    idx[::100] += 1 << 32
+    ms.append(_best_ms(lambda: handle.gather(src, idx, dst)))
+    print(ms)
+    assert ms[1] < 1.7 * ms[0]
+
+
 def test_gather_on_changing_streams(handle):
     """Two streams in turn: the scratch of one call is not written by the next
     before it is read."""
