@@ -64,7 +64,7 @@ hipError_t Arena::get(int slot, size_t bytes, hipStream_t stream, void** out) {
     hipError_t e = hipMalloc(&ptr_[slot], want);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      e = hipMalloc(&ptr_[slot], bytes);
+      e = slot == kGather ? hipMalloc(&ptr_[slot], bytes) : allocate(&ptr_[slot], bytes);
       if (e != hipSuccess) {
         ptr_[slot] = nullptr;
         (void)hipGetLastError();
@@ -77,6 +77,19 @@ hipError_t Arena::get(int slot, size_t bytes, hipStream_t stream, void** out) {
   }
   *out = ptr_[slot];
   return hipSuccess;
+}
+
+hipError_t Arena::allocate(void** out, size_t bytes) {
+  hipError_t e = hipMalloc(out, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  std::lock_guard<std::mutex> lock(gather_mutex);
+  if (!ptr_[kGather]) return e;
+  if (gather_done) (void)hipEventSynchronize(gather_done);
+  (void)hipFree(ptr_[kGather]);
+  ptr_[kGather] = nullptr;
+  cap_[kGather] = 0;
+  return hipMalloc(out, bytes);
 }
 
 size_t Arena::bytes() const {
@@ -189,16 +202,16 @@ hipError_t gather_device(gs_handle* h, int elem_bytes, const void* src, const ui
     (void)hipGetLastError();
     return gather_values(elem_bytes, src, idx, dst, n, h->stream);
   }
-  std::lock_guard<std::mutex> lock(h->gather_mutex);
+  std::lock_guard<std::mutex> lock(h->arena.gather_mutex);
   // Allocating must not end a capture under way on another thread.
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   (void)hipThreadExchangeStreamCaptureMode(&mode);
   void* ws = nullptr;
   hipError_t e = hipSuccess;
-  if (h->gather_done == nullptr)
-    e = hipEventCreateWithFlags(&h->gather_done, hipEventDisableTiming);
-  else if (h->stream != h->gather_stream || h->stream != nullptr)  // a stream made anew may have an old one's address
-    e = hipStreamWaitEvent(h->stream, h->gather_done, 0);
+  if (h->arena.gather_done == nullptr)
+    e = hipEventCreateWithFlags(&h->arena.gather_done, hipEventDisableTiming);
+  else if (h->stream != h->arena.gather_stream || h->stream != nullptr)  // a stream made anew may have an old one's address
+    e = hipStreamWaitEvent(h->stream, h->arena.gather_done, 0);
   if (e == hipSuccess) e = h->arena.get(Arena::kGather, bytes, h->stream, &ws);
   (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (e != hipSuccess) {
@@ -206,8 +219,8 @@ hipError_t gather_device(gs_handle* h, int elem_bytes, const void* src, const ui
     return gather_values(elem_bytes, src, idx, dst, n, h->stream);
   }
   e = gather_split(elem_bytes, src, idx, dst, n, ws, h->stream);
-  h->gather_stream = h->stream;
-  const hipError_t rec = hipEventRecord(h->gather_done, h->stream);
+  h->arena.gather_stream = h->stream;
+  const hipError_t rec = hipEventRecord(h->arena.gather_done, h->stream);
   return e != hipSuccess ? e : rec;
 }
 
@@ -464,7 +477,7 @@ gs_status gs_destroy(gs_handle* h) {
     h->arena.release();
     if (h->pinned) (void)hipHostFree(h->pinned);
     h->stage.release();
-    if (h->gather_done) (void)hipEventDestroy(h->gather_done);
+    if (h->arena.gather_done) (void)hipEventDestroy(h->arena.gather_done);
   }
   delete h;
   return GS_OK;

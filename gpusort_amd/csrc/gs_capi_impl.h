@@ -53,6 +53,9 @@ class Arena {
   }
   ~Arena();
   hipError_t get(int slot, size_t bytes, hipStream_t stream, void** out);
+  // hipMalloc for what a call cannot do without: where there is no memory left,
+  // the gather's scratch, which the gather can do without, is given back first.
+  hipError_t allocate(void** out, size_t bytes);
   // Bytes a slot allocates when it must grow to hold `bytes` (1/8 headroom,
   // whole MiB).
   static size_t grown(size_t bytes) {
@@ -62,6 +65,12 @@ class Arena {
   }
   size_t bytes() const;
   void release();
+
+  // The gather's scratch: gathers from several threads queue one after
+  // another, and one on another stream than the last waits for it.
+  std::mutex gather_mutex;
+  hipEvent_t gather_done = nullptr;
+  hipStream_t gather_stream = nullptr;
 
  private:
   void* ptr_[kSlots];
@@ -129,11 +138,6 @@ struct gs_handle {
   // 0: the device's free memory at the call.
   uint64_t host_budget = 0;
   gs::Arena arena;
-  // The gather's scratch: gathers from several threads queue one after
-  // another, and one on another stream than the last waits for it.
-  std::mutex gather_mutex;
-  hipEvent_t gather_done = nullptr;
-  hipStream_t gather_stream = nullptr;
   gs::Profiler profiler;
   gs::LaunchTimer* timer() { return profiler.active ? &profiler : nullptr; }
   void* pinned = nullptr;

@@ -387,8 +387,8 @@ gs_status gs_seg_plan_create(gs_handle* h, gs_dtype kdt, gs_dtype vdt, const uin
   hipError_t e = hipStreamCreate(&p->own_stream);
   std::vector<unsigned char> meta(p->host.meta_bytes);
   fill_seg_meta(&p->host, nseg ? h_offsets : &zero, meta.data());
-  if (e == hipSuccess) e = hipMalloc(&p->d_meta, meta.size());
-  if (e == hipSuccess && p->host.ws_bytes) e = hipMalloc(&p->d_ws, p->host.ws_bytes);
+  if (e == hipSuccess) e = h->arena.allocate(&p->d_meta, meta.size());
+  if (e == hipSuccess && p->host.ws_bytes) e = h->arena.allocate(&p->d_ws, p->host.ws_bytes);
   if (e == hipSuccess) e = hipMemcpy(p->d_meta, meta.data(), meta.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     (void)hipGetLastError();
@@ -486,10 +486,10 @@ extern "C" gs_status gs_autotune_segments(gs_handle* h, gs_dtype kdt, gs_dtype v
   const uint64_t n = off.back();
   const uint32_t nseg = (uint32_t)off.size() - 1;
   void *k0 = nullptr, *k1 = nullptr, *v0 = nullptr, *v1 = nullptr;
-  hipError_t e = hipMalloc(&k0, n * kb);
-  if (e == hipSuccess) e = hipMalloc(&k1, n * kb);
-  if (e == hipSuccess && vb) e = hipMalloc(&v0, n * vb);
-  if (e == hipSuccess && vb) e = hipMalloc(&v1, n * vb);
+  hipError_t e = h->arena.allocate(&k0, n * kb);
+  if (e == hipSuccess) e = h->arena.allocate(&k1, n * kb);
+  if (e == hipSuccess && vb) e = h->arena.allocate(&v0, n * vb);
+  if (e == hipSuccess && vb) e = h->arena.allocate(&v1, n * vb);
   auto release = [&]() {
     hipFree(k0);
     hipFree(k1);

@@ -317,8 +317,11 @@ gs_status gs_vrank_sort_host(gs_handle* h, gs_algorithm algo, gs_dtype kdt, void
 
 /* dst[i] = src[idx[i]] for a payload of elem_bytes (1, 2, 4, 8) bytes.
  * Device form of ParUtils::ArrangeValues (include/par/par_utils.h:22-86).
- * From 2^24 elements it takes 6 bytes an element of the handle's arena (none
- * under stream capture or where they cannot be had: it is slower then). */
+ * From 2^24 elements it takes 6.1 bytes an element of the handle's arena (up to
+ * an eighth more where there is room; none under stream capture or where they
+ * cannot be had: it is slower then).  The arena keeps them until
+ * gs_release_arena, gs_destroy, or another call on the handle that finds no
+ * device memory. */
 gs_status gs_gather(gs_handle* h, int elem_bytes, const void* d_src, const uint64_t* d_idx, void* d_dst,
                     uint64_t n);
 
