@@ -123,10 +123,9 @@ uint32_t radix_seg_tile_keys(int key_bytes, int val_bytes, int geo);
 int radix_seg_large_geo(int key_bytes, int val_bytes, uint64_t tiles, uint64_t tiles4);
 
 // Size classes of the batched segmented sort: segments of at most small_max
-// keys (<= block_sort_max) are sorted in LDS, those of at
-// most medium_max by the segmented onesweep with the small tiles, the rest in
-// LDS where they fit one tile (block_sort_tile_max) and with the large tiles
-// where not.
+// keys (<= block_sort_max) are sorted in LDS, those of at most medium_max by the
+// segmented onesweep with the small tiles, the rest with the large tiles, or, where
+// small_max is at its limit, in LDS if they fit one tile (block_sort_tile_max).
 struct SegConfig {
   uint32_t small_max;
   uint64_t medium_max;

@@ -5,8 +5,8 @@
 // sequence and one synchronisation per array.  Here every segment of one
 // call is sorted by a fixed number of launches, whatever the count:
 //
-//   small  (<= one LDS tile): one workgroup per segment, sorted in LDS
-//          (block_sort.hip), one launch per length class
+//   small  (<= one LDS tile, or the configured limit): one workgroup per
+//          segment, sorted in LDS (block_sort.hip), one launch per length class
 //   radix  (up to 2^30 keys): segmented onesweep -- one histogram launch,
 //          one scan launch and one launch per digit for all of them; tiles
 //          never straddle segments and the look-back stops at the segment's
@@ -67,8 +67,9 @@ void build_seg_plan(int kb, int vb, const uint64_t* off, uint32_t nseg, const Se
   const uint32_t small_max = std::min<uint32_t>(cfg.small_max, block_sort_max(kb, vb));
   // A segment past the medium class that fits one LDS tile is read and
   // written once there instead of once per digit: 4300 arrays of 4097-16384
-  // pairs 0.41 ms, as part of the large-tile passes about 0.9 ms.
-  const uint64_t tile_max = block_sort_tile_max(kb, vb);
+  // pairs 0.41 ms, as part of the large-tile passes about 0.9 ms.  A lower limit
+  // than the largest is one for these too.
+  const uint64_t tile_max = small_max < block_sort_max(kb, vb) ? small_max : block_sort_tile_max(kb, vb);
   P->grp[0].geo = 0;
   P->grp[1].geo = 1 + (int)std::min<uint32_t>(cfg.medium_geometry, 2u);
   // Where a segment goes depends on its length by thresholds only: they are

@@ -246,8 +246,9 @@ gs_status gs_profile_end(gs_handle* h, gs_kernel_stat* out, uint32_t max_out, ui
 /* Size classes of the batched sort for one (key, payload) width pair:
  * segments of at most small_max keys (at most the LDS tile) are sorted in LDS,
  * one workgroup each, those of at most medium_max by the segmented onesweep
- * with small (4K / 3K-key) tiles, the rest in LDS where one workgroup holds
- * them (up to 9K-16K keys) and with the large tiles where not.  Kept per
+ * with small (4K / 3K-key) tiles, the rest with the large tiles.  With small_max
+ * at its limit (the default) those past medium_max that one workgroup holds (up
+ * to 9K-16K keys) are sorted in LDS as well.  Kept per
  * handle; gs_autotune_segments picks them by measurement.  No counterpart in
  * the reference (one array per call, src/cuda_utils.cu:97-243). */
 typedef struct gs_seg_config {
