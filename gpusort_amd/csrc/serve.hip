@@ -139,7 +139,7 @@ namespace {
 // `count` requests of `total` keys coalesced.
 size_t need_single(gs_dtype kdt, gs_dtype vdt, uint64_t n, bool host) {
   const int kb = dtype_bytes(kdt), vb = val_bytes_of(vdt);
-  size_t b = n <= block_sort_max(kb, vb) ? 0 : Arena::grown(radix_workspace_bytes(kb, vb, n));
+  size_t b = n <= block_sort_tile_max(kb, vb) ? 0 : Arena::grown(radix_workspace_bytes(kb, vb, n));
   if (host) b += Arena::grown((size_t)n * kb) + (vb ? Arena::grown((size_t)n * vb) : 0);  // device staging
   return b;
 }

@@ -203,3 +203,25 @@ def test_slots_overlap_on_the_device(handle):
             handle.sort_pairs(k0, v0)
         torch.cuda.synchronize()
         assert same(req[0], k0) and same(req[1], v0)
+
+
+@pytest.mark.parametrize("kdt,vdt,tile", [(torch.uint32, torch.uint32, 16384), (torch.uint64, torch.uint32, 12288),
+                                          (torch.uint64, torch.uint64, 9216)])
+def test_budget_of_a_request_sorted_in_one_workgroup(kdt, vdt, tile):
+    """Up to one LDS tile a request needs no workspace, so none is reserved: it fits
+    a budget that holds none, and one key more does not."""
+    with g.Server(streams=1, hbm_budget=4096, serial=True) as srv:
+        for n in (tile, 4097, tile + 1):
+            k = torch.randint(0, 1 << 30, (n,), device="cuda", dtype=torch.int64).to(torch.int32 if kdt == torch.uint32 else torch.int64)
+            v = torch.arange(n, device="cuda", dtype=torch.int32 if vdt == torch.uint32 else torch.int64)
+            want = torch.sort(k, stable=True)
+            torch.cuda.synchronize()
+            if n > tile:
+                with pytest.raises(g.GpusortError) as e:
+                    srv.submit(k.view(kdt), v.view(vdt))
+                assert e.value.status == 3
+                continue
+            assert srv.wait(srv.submit(k.view(kdt), v.view(vdt)), timeout_us=-1)
+            torch.cuda.synchronize()
+            assert torch.equal(k, want[0]) and torch.equal(v.long(), want[1])
+        assert srv.stats()["peak_pooled_bytes"] == 0
