@@ -131,6 +131,7 @@ void PinnedStage::release() {
 // ---------------------------------------------------------------- profiler
 Profiler::~Profiler() {
   for (hipEvent_t e : pool_) (void)hipEventDestroy(e);
+  for (SortCtrl* c : watch_pool_) (void)hipHostFree(c);
 }
 
 hipEvent_t Profiler::take() {
@@ -143,7 +144,7 @@ hipEvent_t Profiler::take() {
 }
 
 void Profiler::begin(const char* name, uint64_t bytes, hipStream_t stream) {
-  Rec r{name, bytes, take(), nullptr};
+  Rec r{name, bytes, take(), nullptr, nullptr, 0};
   if (r.start) (void)hipEventRecord(r.start, stream);
   recs.push_back(r);
 }
@@ -155,9 +156,39 @@ void Profiler::end(hipStream_t stream) {
   if (r.stop) (void)hipEventRecord(r.stop, stream);
 }
 
+const SortCtrl* Profiler::watch(const SortCtrl* d_ctrl, hipStream_t stream) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (watch_used_ == watch_pool_.size() * kWatchBlock) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kWatchBlock * sizeof(SortCtrl), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    watch_pool_.push_back(static_cast<SortCtrl*>(p));
+  }
+  SortCtrl* const at = watch_pool_[watch_used_ / kWatchBlock] + watch_used_ % kWatchBlock;
+  if (hipMemcpyAsync(at, d_ctrl, sizeof(SortCtrl), hipMemcpyDeviceToHost, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  ++watch_used_;
+  return at;
+}
+
+void Profiler::only_if(const SortCtrl* watched, int pass) {
+  if (recs.empty()) return;
+  recs.back().watched = watched;
+  recs.back().pass = pass;
+}
+
 void Profiler::reset() {
   recs.clear();
   used_ = 0;
+  watch_used_ = 0;
 }
 
 DeviceScope::DeviceScope(int dev) {
@@ -716,6 +747,7 @@ gs_status gs_profile_end(gs_handle* h, gs_kernel_stat* out, uint32_t max_out, ui
   for (const auto& r : h->profiler.recs) {
     float ms = 0.f;
     if (!r.start || !r.stop || hipEventElapsedTime(&ms, r.start, r.stop) != hipSuccess) continue;
+    if (!r.ran()) continue;
     gs_kernel_stat* st = nullptr;
     for (auto& a : agg)
       if (r.name == a.name) st = &a;

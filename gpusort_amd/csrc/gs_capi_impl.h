@@ -24,17 +24,32 @@ class Profiler : public LaunchTimer {
     std::string name;
     uint64_t bytes;
     hipEvent_t start, stop;
+    const SortCtrl* watched;  // pinned, filled before `start`; null: it counts
+    int pass;
+    // Whether the launch did its work (once its stop event has passed).
+    bool ran() const {
+      if (!watched) return true;
+      if (pass == kTiePass) return watched->low() != 0;
+      return watched->src[pass] == kSkipPass ? false
+             : watched->src[pass] & kCopyPass ? true
+                                              : (uint32_t)pass >= watched->low();
+    }
   };
   ~Profiler() override;
   void begin(const char* name, uint64_t bytes, hipStream_t stream) override;
   void end(hipStream_t stream) override;
+  const SortCtrl* watch(const SortCtrl* d_ctrl, hipStream_t stream) override;
+  void only_if(const SortCtrl* watched, int pass) override;
   void reset();
   std::vector<Rec> recs;
   bool active = false;
 
  private:
+  static constexpr size_t kWatchBlock = 128;
   std::vector<hipEvent_t> pool_;
   size_t used_ = 0;
+  std::vector<SortCtrl*> watch_pool_;  // pinned, kWatchBlock each
+  size_t watch_used_ = 0;
   hipEvent_t take();
 };
 

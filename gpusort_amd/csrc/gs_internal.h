@@ -65,6 +65,13 @@ class LaunchTimer {
   virtual ~LaunchTimer() {}
   virtual void begin(const char* name, uint64_t bytes, hipStream_t stream) = 0;
   virtual void end(hipStream_t stream) = 0;
+  // For launches that leave at once where the device's control block says so:
+  // watch() queues a copy of the block as it is then; the last begun launch
+  // counts only if that copy says that pass `pass` runs (kTiePass: that digits
+  // were left out).  Null (under capture, no memory): it counts.
+  static constexpr int kTiePass = -1;
+  virtual const SortCtrl* watch(const SortCtrl* d_ctrl, hipStream_t stream) = 0;
+  virtual void only_if(const SortCtrl* watched, int pass) = 0;
 };
 
 // Tile hand-out of the onesweep passes.  Grouped hand-out (consecutive tiles

@@ -1245,6 +1245,7 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
                        xf, ctrl, hist, reinterpret_cast<uint4*>(status), status_bytes / 16);
   if (timer) timer->end(stream);
   hipLaunchKernelGGL(radix_scan_kernel, dim3(1), dim3(256), 0, stream, hist, base, ctrl, L.passes, n);
+  const SortCtrl* const watched = timer && sizeof(U) == 8 ? timer->watch(ctrl, stream) : nullptr;
   for (int p = 0; p < L.passes; ++p) {
     OnesweepArgs<U, V, S> a;
     a.keys0 = keys;
@@ -1260,7 +1261,10 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
     a.ctrl = ctrl;
     a.tiles = (uint32_t)L.tiles;
     a.group = tile_group(stream, policy);
-    if (timer) timer->begin("onesweep_pass", 2 * n * (sizeof(U) + (KV ? sizeof(V) : 0)), stream);
+    if (timer) {
+      timer->begin("onesweep_pass", 2 * n * (sizeof(U) + (KV ? sizeof(V) : 0)), stream);
+      timer->only_if(watched, p);
+    }
     if (ident)
       hipLaunchKernelGGL((onesweep_kernel<U, V, KV, THREADS, ITEMS, S, true, false, Idx>), dim3((uint32_t)L.tiles),
                          dim3(THREADS), 0, stream, a);
@@ -1281,7 +1285,7 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
     t.template use_status<THREADS * ITEMS, KV>(status, L.tiles);
     // One chunk a workgroup up to 2^23 keys (four a CU at 2^21), then four.
     t.tile_keys = n <= (1ull << 23) ? kTieChunk : 4 * kTieChunk;
-    launch_tie_fix<V, KV, S>(t, (n + t.tile_keys - 1) / t.tile_keys, n, stream, timer);
+    launch_tie_fix<V, KV, S>(t, (n + t.tile_keys - 1) / t.tile_keys, n, stream, timer, watched);
   }
   return hipGetLastError();
 }
@@ -1560,6 +1564,7 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
     hipLaunchKernelGGL((seg_hist_kernel<U, false, 256>), hist_grid, dim3(256), 0, stream, h);
   if (timer) timer->end(stream);
   hipLaunchKernelGGL(seg_scan_kernel, dim3(T.nslots), dim3(256), 0, stream, cnt, L.passes, ctrl);
+  const SortCtrl* const watched = timer && sizeof(U) == 8 ? timer->watch(ctrl, stream) : nullptr;
   for (int p = 0; p < L.passes; ++p) {
     OnesweepArgs<U, V, uint32_t> a{};
     a.keys0 = keys;
@@ -1580,7 +1585,10 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
     a.seg_base = cnt;
     a.passes = L.passes;
     a.group = tile_group(stream, policy);
-    if (timer) timer->begin("seg_onesweep_pass", 2 * T.n_keys * (sizeof(U) + (KV ? sizeof(V) : 0)), stream);
+    if (timer) {
+      timer->begin("seg_onesweep_pass", 2 * T.n_keys * (sizeof(U) + (KV ? sizeof(V) : 0)), stream);
+      timer->only_if(watched, p);
+    }
     if (ident)
       hipLaunchKernelGGL((onesweep_kernel<U, V, KV, THREADS, ITEMS, uint32_t, true, true, Idx>),
                          dim3((uint32_t)T.tiles), dim3(THREADS), 0, stream, a);
@@ -1603,7 +1611,7 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
       t.seg_first = T.seg_first;
       t.seg_range = T.seg_range;
       t.template use_status<THREADS * ITEMS, KV>(status, T.tiles);
-      launch_tie_fix<V, KV, uint32_t>(t, T.tiles, T.n_keys, stream, timer);
+      launch_tie_fix<V, KV, uint32_t>(t, T.tiles, T.n_keys, stream, timer, watched);
     }
   }
   return hipGetLastError();

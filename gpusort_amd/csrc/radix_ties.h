@@ -720,9 +720,18 @@ __global__ __launch_bounds__(1024) void long_run_kernel(TieArgs<V> a) {
 }
 
 template <typename V, bool KV, typename S>
-void launch_tie_fix(const TieArgs<V>& t, uint64_t tiles, uint64_t n_keys, hipStream_t stream, LaunchTimer* timer) {
-  if (timer) timer->begin("tie_fix", n_keys * 8, stream);
+void launch_tie_fix(const TieArgs<V>& t, uint64_t tiles, uint64_t n_keys, hipStream_t stream, LaunchTimer* timer,
+                    const SortCtrl* watched) {
+  if (timer) {
+    timer->begin("tie_fix", n_keys * 8, stream);
+    timer->only_if(watched, LaunchTimer::kTiePass);
+  }
   hipLaunchKernelGGL((tie_fix_kernel<V, KV>), dim3((uint32_t)tiles), dim3(256), 0, stream, t);
+  if (timer) {
+    timer->end(stream);
+    timer->begin("long_run", 0, stream);  // its bytes depend on the keys
+    timer->only_if(watched, LaunchTimer::kTiePass);
+  }
   hipLaunchKernelGGL((long_run_kernel<V, KV, S>), dim3((uint32_t)std::min<uint64_t>(256, n_keys / 16384 + 1)),
                      dim3(1024), 0, stream, t);
   if (timer) timer->end(stream);

@@ -229,7 +229,8 @@ gs_status gs_generate(gs_handle* h, int dist, uint64_t seed, void* d_out, uint64
  * handle launches for a sort is bracketed by events on its stream;
  * gs_profile_end synchronises and returns per-kernel aggregates.  Bytes are
  * the algorithmic HBM bytes of the launches (one read of the inputs, one
- * write of the outputs).  Counterpart of the reference's phase timers
+ * write of the outputs); the passes that a sort of 64-bit keys leaves out are
+ * not counted.  Counterpart of the reference's phase timers
  * (src/cuda_utils.cu:29-34, src/timer.cc:24-32). */
 typedef struct gs_kernel_stat {
   char name[48];
