@@ -925,6 +925,15 @@ struct Geometry<uint64_t, 8> {
 // 13) -> 81, u32 + i64 69 -> 57.  Past max_rounds the larger
 // tile's shorter look-back weighs more (12 M u32 + u32: 279 with 19, 283 with
 // 16; 67 M 1247, 1261); up to tiny_max the last one is taken.
+//
+// Both sides of those lines, every tile forced in turn (us):
+//   tiny_max, the last tile and the one before it: u32 1.0 M 76 77, 2.1 M 106 89;
+//   u32 + u32 0.39 M 62 65, 0.59 M 70 71, 1.6 M 111 94; u32 + i64 1.0 M 92 90, 1.3
+//   M 100 92; u64 0.26 M 75 76, 0.52 M 85 86, 1.0 M 108 100; u64 + u32 1.0 M 114
+//   116, 1.3 M 126 119; u64 + i64 0.52 M 94 101, 0.79 M 110 108.
+//   max_rounds, the smallest tile of as many rounds and the large one: u32 1.5
+//   rounds 195 201, 2.6 279 292, 4.3 427 442, 6.5 599 586; u32 + u32 1.5 rounds 176
+//   181, 2.1 231 233, 3.2 308 306; u64 0.25 rounds 100 111, 1.1 209 184.
 struct SortTile {
   int threads, items;
 };

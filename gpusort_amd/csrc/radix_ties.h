@@ -98,66 +98,77 @@ __device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint6
   // (256 times as many with every digit, up to the whole sample), and the lowest
   // low at which the samples on both sides agree.
   float ties[4];
-  uint32_t same[4];
-  uint64_t* const ends = reinterpret_cast<uint64_t*>(t.counts());  // a bit for every sample whose next one differs
+  uint32_t next[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const uint32_t p = tid + (uint32_t)j * 256;
     ties[j] = 0.0f;
-    same[j] = 8;
-    const uint64_t a = sk[p], b = sk[p + 1 < kLowSample ? p + 1 : p];
-    if (a != b) {
+    next[j] = 8;
+    if (p + 1 < kLowSample) {
       // The staged samples are in order but for a few neighbours: those count
       // as close ones.
-      ties[j] = per * __builtin_amdgcn_rcpf(b > a ? (float)(b - a) : 1.0f);
-      same[j] = 8 - (uint32_t)__clzll((long long)(a ^ b)) / 8;
-    }
-    const uint64_t w = ballot(a != b);
-    if ((tid & 63u) == 0) ends[p / 64] = w;
-  }
-  lds_barrier();
-  // Equal samples that end at this thread's places: how many, and the lowest low
-  // at which they agree with different ones before or after them.
-  uint32_t size[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t p = tid + (uint32_t)j * 256;
-    size[j] = 0;
-    if (ties[j] == 0.0f && p + 1 < kLowSample) continue;
-    int w = (int)(p / 64);
-    uint64_t before = ends[w] & ((1ull << (p % 64)) - 1);
-    while (before == 0 && w > 0) before = ends[--w];
-    const int last = before ? w * 64 + 63 - __clzll((long long)before) : -1;
-    size[j] = (uint32_t)((int)p - last);
-    if (last >= 0) {
-      const uint32_t above = 8 - (uint32_t)__clzll((long long)(sk[last] ^ sk[last + 1])) / 8;
-      same[j] = same[j] | (above << 8);
-    } else {
-      same[j] |= 8u << 8;
+      const uint64_t a = sk[p], b = sk[p + 1];
+      if (a != b) {
+        ties[j] = per * __builtin_amdgcn_rcpf(b > a ? (float)(b - a) : 1.0f);
+        next[j] = 8 - (uint32_t)__clzll((long long)(a ^ b)) / 8;
+      }
     }
   }
 #pragma unroll
   for (uint32_t low = 1; low < 8; ++low) {
     if (!((allowed >> low) & 1u)) continue;
     float sum = 0.0f;
-    uint32_t mixed = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t next = same[j] & 0xFFu, prev = same[j] >> 8;
-      if (next > low) sum += fminf(ties[j] * (float)(1ull << (8 * low)), 4096.0f);
-      if (next <= low || prev <= low) mixed += size[j];
-    }
-    const uint32_t w = wave_incl_scan_dpp((uint32_t)sum), m = wave_incl_scan_dpp(mixed);
-    if ((tid & 63u) == 63u) {
-      atomicAdd(&s_sum[low], w + 4096u * m);
-      atomicAdd(&s_sum[8 + low], m);
-    }
+    for (int j = 0; j < 4; ++j) sum += fminf(ties[j] * (float)(1ull << (8 * low)), 4096.0f);
+    const uint32_t w = wave_incl_scan_dpp((uint32_t)sum);
+    if ((tid & 63u) == 63u) atomicAdd(&s_sum[low], w);
   }
   lds_barrier();
-  for (uint32_t low = 7; low > 0; --low)
-    if (((allowed >> low) & 1u) && s_sum[low] <= 4096u * kLowSample / kTieFrac &&
-        (n >= kSharedMin || s_sum[8 + low] * n <= (uint64_t)kLdsRun * kLowSample))
-      return low;
+  constexpr uint32_t kMost = 4096u * kLowSample / kTieFrac;
+  uint32_t prev[4], size[4];
+  bool sized = false;
+  for (uint32_t low = 7; low > 0; --low) {
+    if (!((allowed >> low) & 1u) || s_sum[low] > kMost) continue;
+    uint32_t pairs = 0;  // different samples side by side in one run
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pairs += next[j] <= low ? 1u : 0u;
+    if (!__syncthreads_or((int)pairs)) return low;
+    if (!sized) {
+      // Equal samples that end at this thread's places: how many, and the lowest
+      // low at which they agree with the different ones before them.
+      sized = true;
+      uint64_t* const ends = reinterpret_cast<uint64_t*>(t.counts());  // a bit for every sample whose next one differs
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint64_t w = ballot(ties[j] != 0.0f);
+        if ((tid & 63u) == 0) ends[(tid + (uint32_t)j * 256) / 64] = w;
+      }
+      lds_barrier();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t p = tid + (uint32_t)j * 256;
+        prev[j] = 8;
+        size[j] = 0;
+        if (ties[j] == 0.0f && p + 1 < kLowSample) continue;
+        int w = (int)(p / 64);
+        uint64_t before = ends[w] & ((1ull << (p % 64)) - 1);
+        while (before == 0 && w > 0) before = ends[--w];
+        const int last = before ? w * 64 + 63 - __clzll((long long)before) : -1;
+        size[j] = (uint32_t)((int)p - last);
+        if (last >= 0) prev[j] = 8 - (uint32_t)__clzll((long long)(sk[last] ^ sk[last + 1])) / 8;
+      }
+    }
+    uint32_t mixed = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mixed += next[j] <= low || prev[j] <= low ? size[j] : 0u;
+    const uint32_t m = wave_incl_scan_dpp(mixed), c = wave_incl_scan_dpp(pairs);
+    if ((tid & 63u) == 63u) {
+      atomicAdd(&s_sum[8 + low], m);
+      atomicAdd(&s_sum[low], 4096u * (m - c));  // such a pair counted as one
+    }
+    lds_barrier();
+    if (s_sum[low] <= kMost && (n >= kSharedMin || s_sum[8 + low] * n <= (uint64_t)kLdsRun * kLowSample)) return low;
+  }
   return 0;
 }
 
@@ -436,6 +447,8 @@ __global__ __launch_bounds__(1024) void long_run_kernel(TieArgs<V> a) {
   __shared__ uint32_t s_task;
   SortCtrl* const ctrl = a.ctrl;
   const uint32_t count = ctrl->long_count, low = ctrl->low();
+  const uint32_t runs = (uint32_t)(ctrl->shared >> 32), chunks = (uint32_t)ctrl->shared;
+  if (count == 0 && chunks == 0) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const int s = 8 * (int)low;
   uint64_t* const keys = a.keys0;
@@ -471,7 +484,6 @@ __global__ __launch_bounds__(1024) void long_run_kernel(TieArgs<V> a) {
     __syncthreads();
   }
 
-  const uint32_t runs = (uint32_t)(ctrl->shared >> 32), chunks = (uint32_t)ctrl->shared;
   if (chunks == 0) return;
   S* const rows = reinterpret_cast<S*>(a.rows_end) - (uint64_t)chunks * 256;
   // A task takes `group` chunks, so that a phase is about one task a workgroup.
