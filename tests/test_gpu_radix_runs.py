@@ -59,7 +59,7 @@ def _keys(name: str, n: int, seed: int) -> np.ndarray:
     raise ValueError(name)
 
 
-CASES = [("hot", (1 << 22) + 5), ("several", (1 << 22) + 11), ("sentinel1", 1 << 18), ("sentinel2", (1 << 18) + 4097),
+CASES = [("hot", (1 << 23) + 5), ("several", (1 << 23) + 11), ("hot", 1 << 20), ("sentinel1", 1 << 18), ("sentinel2", (1 << 18) + 4097),
          ("sentinel3", 300_001), ("small", 200_003), ("sentinel2", (1 << 22) + 9), ("sentinels", 5_000_011)]
 
 
@@ -83,7 +83,7 @@ def test_runs_past_a_tile(handle, name, n, vdt):
 
 @pytest.mark.parametrize("vdt", [None, np.uint32, np.uint64], ids=lambda t: "none" if t is None else np.dtype(t).name)
 def test_runs_in_segments(handle, vdt):
-    parts = [_keys("several", (1 << 22) + 3, 1), _keys("uniform", 20_000, 2), _keys("hot", 1 << 22, 3),
+    parts = [_keys("several", (1 << 23) + 3, 1), _keys("uniform", 20_000, 2), _keys("hot", 1 << 23, 3),
              _keys("uniform", 13_000, 4), _keys("sentinel3", 120_001, 5), _keys("uniform", 777, 6)]
     off = np.concatenate([[0], np.cumsum([p.size for p in parts])]).astype(np.uint64)
     keys = np.concatenate(parts)
@@ -98,6 +98,69 @@ def test_runs_in_segments(handle, vdt):
             assert_bits_equal(gk[a:b], keys[a:b][order], f"keys of [{a}, {b})")
             if vals is not None:
                 assert_bits_equal(gv[a:b], vals[a:b][order], f"payloads of [{a}, {b})")
+
+
+def test_runs_in_a_graph_and_without_allocation(handle):
+    """A plan's captured graph replayed between eager sorts (the tasks' counters start
+    from zero every time), and the entry whose workspace is a fixed array."""
+    import torch
+    from gpusort_amd import U32, U64
+
+    parts = [_keys("sentinel3", 400_003, 5), _keys("uniform", 30_000, 6), _keys("sentinels", 300_000, 7)]
+    off = np.concatenate([[0], np.cumsum([p.size for p in parts])]).astype(np.uint64)
+    keys = np.concatenate(parts)
+    vals = np.arange(keys.size, dtype=np.uint32)
+    order = np.concatenate([int(a) + stable_order(keys[int(a):int(b)]) for a, b in zip(off, off[1:])]).astype(np.int64)
+    k0, v0 = dev(keys), dev(vals)
+    tk, tv = k0.clone(), v0.clone()
+    torch.cuda.synchronize()
+    plan = handle.seg_plan(off, U64, U32)
+    try:
+        for replay in range(4):
+            tk.copy_(k0)
+            tv.copy_(v0)
+            torch.cuda.synchronize()
+            say(f"runs in a graph, replay {replay}")
+            plan.launch_graph(tk, tv)
+            torch.cuda.synchronize()
+            assert_bits_equal(host(tk), keys[order], "keys")
+            assert_bits_equal(host(tv), vals[order], "payloads")
+            ek = dev(parts[0])
+            handle.sort_keys(ek)
+            assert_bits_equal(host(ek), np.sort(parts[0]), "eager keys")
+    finally:
+        plan.close()
+    one = parts[0]
+    tk, tv = dev(one), dev(np.arange(one.size, dtype=np.uint32))
+    say("runs without allocation")
+    assert handle.lib.gs_sort_pairs_noalloc(handle.h, U64, tk.data_ptr(), U32, tv.data_ptr(), one.size, 0) == 0
+    torch.cuda.synchronize()
+    assert_bits_equal(host(tv), stable_order(one).astype(np.uint32), "payloads")
+
+
+def test_runs_on_several_streams_at_once():
+    """Handles on streams of their own sort at the same time, each with runs that its
+    workgroups share: no sort waits for another one's workgroups."""
+    import torch
+    import gpusort_amd
+
+    n, m = 500_009, 4
+    keys = [_keys(("sentinels", "sentinel3", "sentinel1", "sentinel2")[i], n + i, i) for i in range(m)]
+    streams = [torch.cuda.Stream() for _ in range(m)]
+    handles = [gpusort_amd.Handle(0, stream=s) for s in streams]
+    base = [dev(k) for k in keys]
+    work = [[b.clone() for b in base] for _ in range(6)]
+    torch.cuda.synchronize()
+    say("runs on several streams")
+    for turn in work:
+        for h, w in zip(handles, turn):
+            h.sort_keys(w)
+    torch.cuda.synchronize()
+    for turn in work:
+        for w, k in zip(turn, keys):
+            assert_bits_equal(host(w), np.sort(k), "keys")
+    for h in handles:
+        h.close()
 
 
 def _best_ms(call, prepare) -> float:
