@@ -242,23 +242,19 @@ __device__ inline bool scan_digits(const unsigned long long* __restrict__ hist, 
 }
 
 // First launch of a sort: zeroes the digit histograms and, with `keys` (64-bit
-// keys, block 0), picks the lowest digit to sort by.
-__global__ __launch_bounds__(256) void radix_prep_kernel(uint32_t* __restrict__ g_hist, uint32_t words, SortCtrl* ctrl,
-                                                         const uint64_t* __restrict__ keys, uint64_t n,
-                                                         Xform<uint64_t> xf) {
-  __shared__ LowTile::Smem s_tile;
-  __shared__ uint32_t s_sum[16];
+// keys, block 0), picks the lowest digit to sort by from S of them.
+template <uint32_t S>
+__global__ __launch_bounds__(LowTileOf<S>::THREADS) void radix_prep_kernel(uint32_t* __restrict__ g_hist,
+                                                                           uint32_t words, SortCtrl* ctrl,
+                                                                           const uint64_t* __restrict__ keys,
+                                                                           uint64_t n, Xform<uint64_t> xf) {
+  __shared__ typename LowTileOf<S>::T::Smem s_tile;
+  __shared__ uint32_t s_sum[24];
+  constexpr uint32_t THREADS = LowTileOf<S>::THREADS;
   const uint32_t tid = threadIdx.x;
-  for (uint32_t i = blockIdx.x * 256 + tid; i < words; i += gridDim.x * 256) g_hist[i] = 0;
+  for (uint32_t i = blockIdx.x * THREADS + tid; i < words; i += gridDim.x * THREADS) g_hist[i] = 0;
   if (blockIdx.x != 0) return;
-  uint32_t low = 0;
-  if (keys) {
-    uint64_t k[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      k[i] = to_ordered(keys[sample_pos((tid >> 6) * 256 + (uint32_t)i * 64 + (tid & 63u), n)], xf);
-    low = choose_low(s_tile, k, n, false, s_sum);
-  }
+  const uint32_t low = keys ? choose_low<S>(s_tile, keys, n, xf, false, s_sum) : 0;
   if (tid < kTieWords) (&ctrl->top_digits)[tid] = tid == 0 && low ? 8 - low : 0;
 }
 
@@ -1224,13 +1220,26 @@ static hipError_t radix_sort_t(U* keys, void* vals_v, uint64_t n, const XformPar
   S* status = reinterpret_cast<S*>(ws + L.off_status);
   const uint64_t status_per_pass = L.tiles * kRadix;
 
-  if constexpr (sizeof(U) == 8)
-    hipLaunchKernelGGL(radix_prep_kernel, dim3(8), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
-                       (uint32_t)(kMaxPasses * kRadix * 2), ctrl, n >= 4 * kLowSample ? (const U*)keys : nullptr, n, xf);
-  else
-    hipLaunchKernelGGL(radix_prep_kernel, dim3(8), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
-                       (uint32_t)(kMaxPasses * kRadix * 2), ctrl, (const uint64_t*)nullptr, n,
-                       Xform<uint64_t>{0, 0, 0});
+  constexpr uint32_t hist_words = kMaxPasses * kRadix * 2;
+  uint32_t* const hist32 = reinterpret_cast<uint32_t*>(hist);
+  if constexpr (sizeof(U) == 8) {
+    const U* const sampled = n >= 4 * kLowSample ? keys : nullptr;
+    if (n >= kLowSample8Min)
+      hipLaunchKernelGGL(radix_prep_kernel<8 * kLowSample>, dim3(2), dim3(1024), 0, stream, hist32, hist_words, ctrl,
+                         sampled, n, xf);
+    else if (n >= kLowSample4Min)
+      hipLaunchKernelGGL(radix_prep_kernel<4 * kLowSample>, dim3(2), dim3(1024), 0, stream, hist32, hist_words, ctrl,
+                         sampled, n, xf);
+    else if (n >= kLowSample2Min)
+      hipLaunchKernelGGL(radix_prep_kernel<2 * kLowSample>, dim3(4), dim3(512), 0, stream, hist32, hist_words, ctrl,
+                         sampled, n, xf);
+    else
+      hipLaunchKernelGGL(radix_prep_kernel<kLowSample>, dim3(8), dim3(256), 0, stream, hist32, hist_words, ctrl,
+                         sampled, n, xf);
+  } else {
+    hipLaunchKernelGGL(radix_prep_kernel<kLowSample>, dim3(8), dim3(256), 0, stream, hist32, hist_words, ctrl,
+                       (const uint64_t*)nullptr, n, Xform<uint64_t>{0, 0, 0});
+  }
   const uint64_t status_bytes = (uint64_t)L.passes * status_per_pass * sizeof(S);
   const uint64_t hist_blocks = hist_blocks_for(n);
   // The histogram kernel counts every key byte (L.passes == sizeof(U)).
@@ -1453,21 +1462,19 @@ __global__ __launch_bounds__(THREADS) void seg_hist_kernel(SegHistArgs<U> a) {
 // or six digits, so that the result lands where the keys were): the largest
 // number of digits counts.  A segment of fewer keys than four samples has no
 // say: all of it fits one workgroup's tile if its keys agree above.
-__global__ __launch_bounds__(256) void seg_prep_kernel(SortCtrl* ctrl, const uint64_t* __restrict__ keys,
-                                                       const uint64_t* __restrict__ seg_range, Xform<uint64_t> xf) {
-  __shared__ LowTile::Smem s_tile;
-  __shared__ uint32_t s_sum[16];
-  const uint32_t tid = threadIdx.x;
+template <uint32_t S>
+__global__ __launch_bounds__(LowTileOf<S>::THREADS) void seg_prep_kernel(SortCtrl* ctrl,
+                                                                         const uint64_t* __restrict__ keys,
+                                                                         const uint64_t* __restrict__ seg_range,
+                                                                         Xform<uint64_t> xf) {
+  __shared__ typename LowTileOf<S>::T::Smem s_tile;
+  __shared__ uint32_t s_sum[24];
   const uint64_t start = seg_range[2 * blockIdx.x];
   const uint64_t len = seg_range[2 * blockIdx.x + 1] - start;
-  if (len < 4 * kLowSample) return;
-  uint64_t k[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    k[i] = to_ordered(keys[start + sample_pos((tid >> 6) * 256 + (uint32_t)i * 64 + (tid & 63u), len)], xf);
-  uint32_t low = choose_low(s_tile, k, len, true, s_sum);
+  if (len < 4 * kLowSample || (len >= kLowSample2Min) != (S > kLowSample)) return;
+  uint32_t low = choose_low<S>(s_tile, keys + start, len, xf, true, s_sum);
   low = low > 4 ? 4 : low;
-  if (tid == 0) atomicMax(&ctrl->top_digits, 8 - low);
+  if (threadIdx.x == 0) atomicMax(&ctrl->top_digits, 8 - low);
 }
 
 // Counts -> exclusive digit starts within the segment, in place, one
@@ -1545,7 +1552,11 @@ static hipError_t radix_segments_t(U* keys, void* vals_v, const SegTiles& T, con
   const bool by_top = sizeof(U) == 8 && T.n_multi != 0;
   if constexpr (sizeof(U) == 8) {
     if (by_top)
-      hipLaunchKernelGGL(seg_prep_kernel, dim3(T.nslots), dim3(256), 0, stream, ctrl, (const U*)keys, T.seg_range, xf);
+      hipLaunchKernelGGL(seg_prep_kernel<kLowSample>, dim3(T.nslots), dim3(256), 0, stream, ctrl, (const U*)keys,
+                         T.seg_range, xf);
+    if (by_top && T.n_keys >= kLowSample2Min)  // a segment may be that long
+      hipLaunchKernelGGL(seg_prep_kernel<2 * kLowSample>, dim3(T.nslots), dim3(512), 0, stream, ctrl, (const U*)keys,
+                         T.seg_range, xf);
   }
   SegHistArgs<U> h;
   h.keys = keys;
@@ -1822,7 +1833,7 @@ static hipError_t multisplit_t(const U* keys, const void* vals, uint64_t n, cons
   unsigned long long* hist = reinterpret_cast<unsigned long long*>(ws + L.off_hist);
   uint64_t* base = d_bucket_base ? d_bucket_base : reinterpret_cast<uint64_t*>(ws + L.off_base);
   S* status = reinterpret_cast<S*>(ws + L.off_status);
-  hipLaunchKernelGGL(radix_prep_kernel, dim3(1), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
+  hipLaunchKernelGGL(radix_prep_kernel<kLowSample>, dim3(1), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(hist),
                      (uint32_t)(kRadix * 2), ctrl, (const uint64_t*)nullptr, n, Xform<uint64_t>{0, 0, 0});
   const uint64_t status_bytes = L.tiles * kRadix * sizeof(S);
   uint64_t blocks = (n + kSplitHistThreads * 16 - 1) / (kSplitHistThreads * 16);

@@ -6,7 +6,7 @@
 // still equal in the sorted bits.  So the passes start at digit `low` (chosen
 // from a sorted sample of the keys, choose_low) and leave short runs of keys
 // that agree from bit 8 * low up, in input order.  tie_fix_kernel reads the
-// keys once and puts runs of up to kShortRun keys in order in place; runs
+// keys once and puts runs of up to kShortRun keys in order by comparing them; runs
 // longer than that with a key out of order (keys that share their high digits:
 // small numbers or a hot prefix among random ones) are listed and sorted by
 // long_run_kernel, in LDS where they fit and by all workgroups together where
@@ -35,20 +35,29 @@
 
 namespace gs {
 
-// Keys of the sample that picks the lowest digit.
+// Keys of the sample that picks the lowest digit, and the least n for twice, four and
+// eight times as many: a sample of S keys shows clusters of r keys that share their
+// high digits by about S^2 r / 2n pairs, and from r = 64 on all digits cost less.
 constexpr uint32_t kLowSample = 1024;
+constexpr uint64_t kLowSample2Min = 1ull << 24, kLowSample4Min = 1ull << 26, kLowSample8Min = 1ull << 28;
 // Digits are added until the sample's ties come to at most 1 in kTieFrac.
 // (Gaps of random keys vary, and 1 / gap is counted: 1 in 8 here is about 1
 // key in 32 that agrees with another one in the sorted bits.)
 constexpr uint32_t kTieFrac = 8;
-constexpr uint32_t kShortRun = 32;
+constexpr uint32_t kShortRun = 256;
 
-using LowTile = BlockRadix<uint64_t, uint32_t, false, 256, 4, false>;
+// The sample in a workgroup.
+template <uint32_t S>
+struct LowTileOf {
+  static constexpr int THREADS = S < 4096 ? S / 4 : 1024, ITEMS = S / THREADS;
+  using T = BlockRadix<uint64_t, uint32_t, false, THREADS, ITEMS, false>;
+};
 
-// Position of sample i of n keys: one in each of kLowSample equal strata, at
-// a place of its own.
+// Position of sample i of S of n keys: one in each of S equal strata, at a place
+// of its own.
+template <uint32_t S>
 __device__ inline uint64_t sample_pos(uint32_t i, uint64_t n) {
-  const uint64_t lo = (uint64_t)i * n / kLowSample, hi = (uint64_t)(i + 1) * n / kLowSample;
+  const uint64_t lo = (uint64_t)i * n / S, hi = (uint64_t)(i + 1) * n / S;
   uint32_t x = i * 0x9E3779B1u;
   x ^= x >> 15;
   x *= 0x85EBCA77u;
@@ -63,25 +72,37 @@ __device__ inline uint64_t sample_pos(uint32_t i, uint64_t n) {
 constexpr uint64_t kSharedMin = 1ull << 23;
 constexpr uint32_t kLdsRun = 4096;
 
-// Lowest digit to sort by, from a sample of the n keys (ordered images in
-// k[], thread t's item i at LowTile::pos): the largest low for which few keys
-// are expected to agree with another one from bit 8 * low up, among those that
-// leave out a digit that varies and leave an even number of varying ones (the
-// result then lands where the keys were); 0 if none.  `even_only`: every digit
-// from low up is a pass, so low itself is even.  The n / kLowSample keys
-// between two neighbouring samples are taken as spread evenly over the gap
-// between them; equal samples are taken as equal keys.  Samples that agree from
-// bit 8 * low up but differ below stand for one run, all of them: half of 2^26
+// Lowest digit to sort by, from a sample of S of the n keys at `keys`: the largest
+// low for which few keys are expected to agree with another one from bit 8 * low
+// up, among those that leave out a digit that varies and leave an even number of
+// varying ones (the result then lands where the keys were); 0 if none.
+// `even_only`: every digit from low up is a pass, so low itself is even.
+//
+// The n / S keys between two neighbouring samples are taken as spread evenly over
+// the gap between them; equal samples are taken as equal keys.  Samples that agree
+// from bit 8 * low up but differ below stand for one run, all of them: half of 2^26
 // keys in 0..99, which as 99 gaps among 1024 looked like few, went to one
-// workgroup (480 ms, by all digits 2.9).  256 threads, all
-// of them; every thread returns the answer.  About 9 us alone on the chip, of
-// which the sample's reads are 2.
-__device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint64_t n, bool even_only,
-                                      uint32_t* s_sum) {
+// workgroup (480 ms, by all digits 2.9).  Two of them with no third stand for many
+// small clusters, of about 2 n / S^2 keys for every such pair: more than kMaxMates
+// keys are more than is worth comparing (2^26 keys in 2^20 clusters: 51 ms).
+//
+// All threads of the workgroup; every one returns the answer.  About 9 us alone on
+// the chip with 1024 samples, of which their reads are 2; 15, 26 and 42 with 2048,
+// 4096 and 8192.
+constexpr uint32_t kMaxMates = 64;
+
+template <uint32_t S>
+__device__ inline uint32_t choose_low(typename LowTileOf<S>::T::Smem& sm, const uint64_t* __restrict__ keys, uint64_t n,
+                                      const Xform<uint64_t>& xf, bool even_only, uint32_t* s_sum) {
+  using LowTile = typename LowTileOf<S>::T;
+  constexpr int THREADS = LowTileOf<S>::THREADS, ITEMS = LowTileOf<S>::ITEMS;
   const uint32_t tid = threadIdx.x;
+  uint64_t k[ITEMS];
   uint32_t none[1];
-  LowTile t{sm, k, none, kLowSample, 4};
-  if (tid < 16) s_sum[tid] = 0;
+  LowTile t{sm, k, none, S, (uint32_t)ITEMS};
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) k[i] = to_ordered(keys[sample_pos<S>(t.pos(i), n)], xf);
+  if (tid < 24) s_sum[tid] = 0;
   const uint64_t diff = t.varying();
   uint32_t allowed = 0, above = 0;
   for (int p = 7; p > 0; --p) {
@@ -93,18 +114,18 @@ __device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint6
   t.sort();
   lds_barrier();
   const uint64_t* const sk = t.keys();
-  const float per = (float)n * (4096.0f / (float)kLowSample);
-  // This thread's four gaps: the ties expected at low = 0, in 1/4096 of a sample
-  // (256 times as many with every digit, up to the whole sample), and the lowest
-  // low at which the samples on both sides agree.
-  float ties[4];
-  uint32_t next[4];
+  const float per = (float)n * (4096.0f / (float)S);
+  // This thread's gaps: the ties expected at low = 0, in 1/4096 of a sample (256
+  // times as many with every digit, up to the whole sample), and the lowest low at
+  // which the samples on both sides agree.
+  float ties[ITEMS];
+  uint32_t next[ITEMS];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t p = tid + (uint32_t)j * 256;
+  for (int j = 0; j < ITEMS; ++j) {
+    const uint32_t p = tid + (uint32_t)j * THREADS;
     ties[j] = 0.0f;
     next[j] = 8;
-    if (p + 1 < kLowSample) {
+    if (p + 1 < S) {
       // The staged samples are in order but for a few neighbours: those count
       // as close ones.
       const uint64_t a = sk[p], b = sk[p + 1];
@@ -119,19 +140,19 @@ __device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint6
     if (!((allowed >> low) & 1u)) continue;
     float sum = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sum += fminf(ties[j] * (float)(1ull << (8 * low)), 4096.0f);
+    for (int j = 0; j < ITEMS; ++j) sum += fminf(ties[j] * (float)(1ull << (8 * low)), 4096.0f);
     const uint32_t w = wave_incl_scan_dpp((uint32_t)sum);
     if ((tid & 63u) == 63u) atomicAdd(&s_sum[low], w);
   }
   lds_barrier();
-  constexpr uint32_t kMost = 4096u * kLowSample / kTieFrac;
-  uint32_t prev[4], size[4];
+  constexpr uint32_t kMost = 4096u * S / kTieFrac;
+  uint32_t prev[ITEMS], size[ITEMS];
   bool sized = false;
   for (uint32_t low = 7; low > 0; --low) {
     if (!((allowed >> low) & 1u) || s_sum[low] > kMost) continue;
     uint32_t pairs = 0;  // different samples side by side in one run
 #pragma unroll
-    for (int j = 0; j < 4; ++j) pairs += next[j] <= low ? 1u : 0u;
+    for (int j = 0; j < ITEMS; ++j) pairs += next[j] <= low ? 1u : 0u;
     if (!__syncthreads_or((int)pairs)) return low;
     if (!sized) {
       // Equal samples that end at this thread's places: how many, and the lowest
@@ -139,17 +160,17 @@ __device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint6
       sized = true;
       uint64_t* const ends = reinterpret_cast<uint64_t*>(t.counts());  // a bit for every sample whose next one differs
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < ITEMS; ++j) {
         const uint64_t w = ballot(ties[j] != 0.0f);
-        if ((tid & 63u) == 0) ends[(tid + (uint32_t)j * 256) / 64] = w;
+        if ((tid & 63u) == 0) ends[(tid + (uint32_t)j * THREADS) / 64] = w;
       }
       lds_barrier();
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t p = tid + (uint32_t)j * 256;
+      for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t p = tid + (uint32_t)j * THREADS;
         prev[j] = 8;
         size[j] = 0;
-        if (ties[j] == 0.0f && p + 1 < kLowSample) continue;
+        if (ties[j] == 0.0f && p + 1 < S) continue;
         int w = (int)(p / 64);
         uint64_t before = ends[w] & ((1ull << (p % 64)) - 1);
         while (before == 0 && w > 0) before = ends[--w];
@@ -158,16 +179,27 @@ __device__ inline uint32_t choose_low(LowTile::Smem& sm, uint64_t (&k)[4], uint6
         if (last >= 0) prev[j] = 8 - (uint32_t)__clzll((long long)(sk[last] ^ sk[last + 1])) / 8;
       }
     }
-    uint32_t mixed = 0;
+    uint32_t mixed = 0, alone = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) mixed += next[j] <= low || prev[j] <= low ? size[j] : 0u;
-    const uint32_t m = wave_incl_scan_dpp(mixed), c = wave_incl_scan_dpp(pairs);
+    for (int j = 0; j < ITEMS; ++j) {
+      mixed += next[j] <= low || prev[j] <= low ? size[j] : 0u;
+      if (next[j] <= low) {  // the pair p, p + 1: has it a third?
+        const uint32_t p = tid + (uint32_t)j * THREADS;
+        const uint64_t g = sk[p] >> (8 * low);
+        alone += (p == 0 || (sk[p - 1] >> (8 * low)) != g) && (p + 2 >= S || (sk[p + 2] >> (8 * low)) != g) ? 1u : 0u;
+      }
+    }
+    const uint32_t m = wave_incl_scan_dpp(mixed), c = wave_incl_scan_dpp(pairs), l = wave_incl_scan_dpp(alone);
     if ((tid & 63u) == 63u) {
-      atomicAdd(&s_sum[8 + low], m);
+      atomicAdd(&s_sum[8 + low], m - 2 * l);
+      atomicAdd(&s_sum[16 + low], l);
       atomicAdd(&s_sum[low], 4096u * (m - c));  // such a pair counted as one
     }
     lds_barrier();
-    if (s_sum[low] <= kMost && (n >= kSharedMin || s_sum[8 + low] * n <= (uint64_t)kLdsRun * kLowSample)) return low;
+    const uint64_t clusters = s_sum[16 + low];
+    if (s_sum[low] <= kMost && (n >= kSharedMin || s_sum[8 + low] * n <= (uint64_t)kLdsRun * S) &&
+        (clusters <= 2 || clusters * n <= (uint64_t)S * S * (kMaxMates / 2)))
+      return low;
   }
   return 0;
 }
@@ -251,49 +283,38 @@ __device__ inline uint64_t first_at_least(const uint64_t* keys, uint64_t lo, uin
 
 // Puts runs of 2..kShortRun keys equal from bit 8 * ctrl->low() up in order,
 // and lists longer runs that hold a key out of order.  A workgroup takes
-// chunks of kTieChunk keys: the chunk is staged in LDS (all loads in flight
-// together) and the positions of keys greater than the key after them in their
-// run are gathered into a list, so that few of them cost one round of the
-// workgroup and equal keys cost nothing.  The thread of a run's first listed
-// position sorts the run.  A run that crosses the chunk's end belongs to the
-// chunk it starts in and is sorted in global memory.  Where a run starts and
-// ends depends only on bits that no step changes, so a run has one owner and
-// reads of other owners' keys decide nothing about it.
+// chunks of kTieChunk keys, staged in LDS with the kShortRun keys behind them (all
+// loads in flight together).  A bit is set for every key that starts a run and for
+// every key greater than the next one of its run; where none of the latter is near,
+// nothing is done, so equal keys cost nothing.  The keys in runs near one are
+// collected, so that the work is by such keys, and each finds the ends of its run
+// from the bits and its place by comparison with all keys of the run.  Payloads are
+// read before any is written.  A run belongs to the chunk it starts in.  Where a run
+// starts and ends depends only on bits that no step changes, so a run has one owner
+// and reads of other owners' keys decide nothing about it.
+//
+// What bounds it: the read of the keys (2^26 random keys, 1.5 % of them in runs, with
+// 32-bit payloads: 200 us); where all keys are in runs of r keys, the r LDS reads
+// a key (r = 4: 0.7 ms, 16: 0.8, 32: 1.0, 64: 1.3).  With a thread a run up to 32
+// keys, in global memory, and a workgroup a run above, the sort of those 2^26 took
+// 13.3 ms at r = 16 and 51 at 64 (now 2.4 and 3.0; by all digits 2.9).  120 registers,
+// four workgroups a CU; five, with two registers spilled, or the next chunk's loads
+// ahead, are slower (keys only: 152 us, 157, 183).
 constexpr uint32_t kTieChunk = 2048;
 
 template <typename V, bool KV>
-__device__ inline void sort_run_serial(uint64_t* keys, V* vals, uint64_t p, uint64_t seg1, uint64_t t, int s,
-                                       const Xform<uint64_t>& xf) {
-  uint32_t len = 2;
-  while (p + len < seg1 && len <= kShortRun && (to_ordered(keys[p + len], xf) >> s) == t) ++len;
-  if (len > kShortRun) return;
-  for (uint32_t i = 1; i < len; ++i) {
-    const uint64_t raw = keys[p + i];
-    const uint64_t x = to_ordered(raw, xf);
-    uint32_t at = i;
-    while (at > 0 && to_ordered(keys[p + at - 1], xf) > x) --at;
-    if (at == i) continue;
-    V y{};
-    if constexpr (KV) y = vals[p + i];
-    for (uint32_t q = i; q > at; --q) {
-      keys[p + q] = keys[p + q - 1];
-      if constexpr (KV) vals[p + q] = vals[p + q - 1];
-    }
-    keys[p + at] = raw;
-    if constexpr (KV) vals[p + at] = y;
-  }
-}
-
-template <typename V, bool KV>
 __global__ __launch_bounds__(256) void tie_fix_kernel(TieArgs<V> a) {
-  constexpr int PER = kTieChunk / 256;
-  __shared__ uint64_t s_k[kTieChunk + 2];  // keys from one before the chunk to one past it
-  __shared__ uint16_t s_tie[kTieChunk];
-  __shared__ uint32_t s_nties;
+  constexpr int PER = (kTieChunk + kShortRun) / 256;
+  constexpr uint32_t PAD = kShortRun / 64, WORDS = (kTieChunk + kShortRun) / 64;
+  static_assert(kShortRun % 256 == 0 && WORDS < 64, "whole rounds of the workgroup, a word a lane");
+  __shared__ uint64_t s_k[kTieChunk + kShortRun + 1];  // from one key before the chunk
+  __shared__ uint64_t s_down[WORDS], s_start[WORDS];
+  __shared__ alignas(16) uint32_t s_any[4];
+  __shared__ uint32_t s_list[kTieChunk + kShortRun];  // place, and the new one in the upper half
   const uint32_t low = a.ctrl->low();
   if (low == 0) return;
   const int s = 8 * (int)low;
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
   uint64_t seg0 = 0, seg1 = a.n, start, end;
   uint32_t slot = 0;
   uint64_t* keys = a.keys0;
@@ -307,83 +328,124 @@ __global__ __launch_bounds__(256) void tie_fix_kernel(TieArgs<V> a) {
     start = (uint64_t)blockIdx.x * a.tile_keys;
   }
   end = start + a.tile_keys < seg1 ? start + a.tile_keys : seg1;
+  // Element i of the chunk.
+  auto at = [&](uint32_t i) -> uint64_t& { return s_k[i + 1]; };
   for (uint64_t c0 = start; c0 < end; c0 += kTieChunk) {
     const uint32_t m = end - c0 < kTieChunk ? (uint32_t)(end - c0) : kTieChunk;
+    const uint32_t staged = seg1 - c0 < m + kShortRun ? (uint32_t)(seg1 - c0) : m + kShortRun;
     uint64_t k[PER];
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const uint32_t i = tid + (uint32_t)j * 256;
-      k[j] = keys[c0 + (i < m ? i : m - 1)];
+      k[j] = keys[c0 + (i < staged ? i : staged - 1)];
     }
-    if (tid == 0) s_nties = 0;
-    // Past the segment's ends: a key of another run.
+    // Before the segment: a key of another run.
     if (tid == 64) s_k[0] = c0 > seg0 ? to_ordered(keys[c0 - 1], a.xf) : ~to_ordered(keys[c0], a.xf);
-    if (tid == 128) s_k[m + 1] = c0 + m < seg1 ? to_ordered(keys[c0 + m], a.xf) : ~to_ordered(keys[c0 + m - 1], a.xf);
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const uint32_t i = tid + (uint32_t)j * 256;
-      if (i < m) s_k[i + 1] = to_ordered(k[j], a.xf);
+      k[j] = to_ordered(k[j], a.xf);
+      if (i < staged) at(i) = k[j];
     }
     lds_barrier();
-    // Element i of the chunk sits at s_k[i + 1].
+    uint64_t down[PER], any = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const uint32_t i = tid + (uint32_t)j * 256;
-      if (i < m) {
-        const uint64_t x = s_k[i + 1], y = s_k[i + 2];
-        if (y < x && (y >> s) == (x >> s)) s_tie[atomicAdd(&s_nties, 1u)] = (uint16_t)i;
+      const uint64_t next = at(i + 1 < staged ? i + 1 : staged - 1);
+      down[j] = ballot(next < k[j] && ((next ^ k[j]) >> s) == 0);
+      any |= down[j];
+    }
+    if (lane == 0) s_any[tid / 64] = any != 0;
+    lds_barrier();
+    const uint4 found = *reinterpret_cast<const uint4*>(s_any);
+    if (__builtin_amdgcn_readfirstlane((int)(found.x | found.y | found.z | found.w)) == 0) continue;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t i = tid + (uint32_t)j * 256;
+      const uint64_t starts = ballot(i >= staged || ((s_k[i] ^ k[j]) >> s) != 0);
+      if (lane == 0) {
+        s_down[i / 64] = down[j];
+        s_start[i / 64] = starts;
       }
     }
     lds_barrier();
-    const uint32_t nties = s_nties;
-    for (uint32_t j = tid; j < nties; j += 256) {
-      const uint32_t i = s_tie[j];
-      const uint64_t t = s_k[i + 1] >> s;
-      // The run's first and last key in the chunk, kShortRun away at most,
-      // and whether an earlier position of it is listed too.
-      uint32_t b = i, e = i + 1;
-      bool first = true;
-      while (b > 0 && i - b <= kShortRun && (s_k[b] >> s) == t) {
-        first &= s_k[b] <= s_k[b + 1];
-        --b;
-      }
-      while (e + 1 < m && e - b <= kShortRun && (s_k[e + 2] >> s) == t) ++e;
-      if (e - b < kShortRun) {
-        if (e >= m || (b == 0 && (s_k[0] >> s) == t) || (e + 1 == m && (s_k[m + 1] >> s) == t)) {
-          // It crosses an end of the chunk: sorted below or by the chunk before.
-        } else if (e == b + 1) {
-          const uint64_t lo = keys[c0 + b], hi = keys[c0 + e];
-          V vl{}, vh{};
-          if constexpr (KV) {
-            vl = vals[c0 + b];
-            vh = vals[c0 + e];
-          }
-          keys[c0 + b] = hi;
-          keys[c0 + e] = lo;
-          if constexpr (KV) {
-            vals[c0 + b] = vh;
-            vals[c0 + e] = vl;
-          }
-          continue;
-        } else {
-          if (first) sort_run_serial<V, KV>(keys, vals, c0 + b, seg1, t, s, a.xf);
-          continue;
+    // A lane a word: the keys of it that are in a run, if a bit is within kShortRun.
+    const uint64_t downs = ballot(lane < WORDS && s_down[lane < WORDS ? lane : 0] != 0);
+    uint64_t in_run = 0;
+    if (lane < WORDS && ((lane >= PAD ? downs >> (lane - PAD) : downs << (PAD - lane)) & ((1u << (2 * PAD + 1)) - 1))) {
+      const uint64_t st = s_start[lane], next = lane + 1 < WORDS ? s_start[lane + 1] : ~0ull;
+      in_run = ~st | ~((st >> 1) | (next << 63));
+    }
+    const uint32_t incl = wave_incl_scan_dpp((uint32_t)__popcll(in_run));
+    const uint32_t count = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t i = tid + (uint32_t)j * 256;
+      const int w = __builtin_amdgcn_readfirstlane((int)(i / 64));
+      const uint64_t bits = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)in_run, w) |
+                            (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(in_run >> 32), w) << 32;
+      const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)incl, w) - (uint32_t)__popcll(bits);
+      if ((bits >> lane) & 1u) s_list[before + (uint32_t)__popcll(bits & ((1ull << lane) - 1))] = i;
+    }
+    lds_barrier();
+    for (uint32_t q = tid; q < count; q += 256) {
+      const uint32_t i = s_list[q];
+      const uint64_t x = at(i), t = x >> s;
+      s_list[q] = i | i << 16;
+      // The run [b, e) as far as it is within kShortRun keys.
+      int w = (int)(i / 64);
+      uint64_t bits = s_start[w] & (~0ull >> (63 - i % 64));
+      for (const int last = w > (int)PAD ? w - (int)PAD : 0; bits == 0 && w > last;) bits = s_start[--w];
+      const bool starts = bits != 0;
+      const uint32_t b = starts ? (uint32_t)(w * 64 + 63 - __clzll((long long)bits)) : 0;
+      w = (int)(i / 64);
+      bits = s_start[w] & ~(~0ull >> (63 - i % 64));
+      for (const int last = w + (int)PAD < (int)WORDS - 1 ? w + (int)PAD : (int)WORDS - 1; bits == 0 && w < last;)
+        bits = s_start[++w];
+      uint32_t e = bits ? (uint32_t)(w * 64) + (uint32_t)__ffsll((unsigned long long)bits) - 1u : staged;
+      if (e > staged) e = staged;
+      // Whether a key of [from, to) is greater than the next of the run.
+      auto unordered = [&](uint32_t from, uint32_t to) {
+        uint64_t found = 0;
+        for (uint32_t v = from / 64; v <= to / 64 && v < WORDS; ++v) {
+          uint64_t d = s_down[v];
+          if (v == from / 64) d &= ~0ull << (from % 64);
+          if (v == to / 64) d &= (1ull << (to % 64)) - 1;
+          found |= d;
         }
+        return found != 0;
+      };
+      if (starts && e - b <= kShortRun) {
+        if (b >= m || !unordered(b, e)) continue;  // the next chunk's
+        uint32_t rank = b;
+#pragma unroll 4
+        for (uint32_t p = b; p < e; ++p) {
+          const uint64_t y = at(p);
+          rank += y < x || (y == x && p < i) ? 1u : 0u;
+        }
+        s_list[q] = i | rank << 16;
+        continue;
       }
-      // Is its run a long one?  (An earlier listed position of it in the chunk
-      // asks for this one too.)
-      if (!first) continue;
-      const uint64_t p = c0 + i;
-      const uint64_t back = p - seg0 > kShortRun ? p - kShortRun : seg0;
-      const uint64_t fwd = seg1 - p > kShortRun + 1 ? p + kShortRun + 1 : seg1;
-      const uint64_t rb = first_at_least(keys, back, p, t, s, a.xf);
-      const uint64_t re = first_at_least(keys, p + 1, fwd, t + 1, s, a.xf);
-      if (re - rb <= kShortRun) continue;
-      const uint64_t run = rb > back ? rb : first_at_least(keys, seg0, rb, t, s, a.xf);
-      // Two runs longer than 32 never start in the same 32 positions.
-      const uint64_t at = a.tile_seg ? (uint64_t)a.seg_first[slot] * a.tile_keys + (run - seg0) : run;
-      const uint32_t bit = 1u << ((at >> 5) & 31u);
-      if (atomicOr(&a.long_seen[at >> 10], bit) & bit) continue;
+      // A long run, or one that starts before the chunk.  An earlier key of it that
+      // is greater than the next asks in its place.
+      if (i >= m || !((s_down[i / 64] >> (i % 64)) & 1u)) continue;
+      const uint32_t seen = starts ? b : i > kShortRun ? (i / 64 - PAD) * 64 : 0;
+      if (unordered(seen, i)) continue;
+      uint64_t run = c0 + b;
+      if (!starts) {
+        const uint64_t p = c0 + i;
+        const uint64_t back = p - seg0 > kShortRun ? p - kShortRun : seg0;
+        const uint64_t fwd = seg1 - p > kShortRun + 1 ? p + kShortRun + 1 : seg1;
+        const uint64_t rb = first_at_least(keys, back, p, t, s, a.xf);
+        const uint64_t re = first_at_least(keys, p + 1, fwd, t + 1, s, a.xf);
+        if (re - rb <= kShortRun) continue;
+        run = rb > back ? rb : first_at_least(keys, seg0, rb, t, s, a.xf);
+      }
+      // Two runs longer than kShortRun never start in the same 32 positions.
+      const uint64_t place = a.tile_seg ? (uint64_t)a.seg_first[slot] * a.tile_keys + (run - seg0) : run;
+      const uint32_t bit = 1u << ((place >> 5) & 31u);
+      if (atomicOr(&a.long_seen[place >> 10], bit) & bit) continue;
       constexpr uint64_t CAP = 1024 * run_items<V, KV>();
       if (seg1 - run > CAP && (to_ordered(keys[run + CAP], a.xf) >> s) == t) {
         const uint64_t len = first_at_least(keys, run + CAP + 1, seg1, t + 1, s, a.xf) - run;
@@ -397,16 +459,25 @@ __global__ __launch_bounds__(256) void tie_fix_kernel(TieArgs<V> a) {
       entry[1] = (uint32_t)(run >> 32);
       entry[2] = slot;
     }
-    // The run that crosses the chunk's end.
-    if (tid == 255) {
-      const uint64_t t = s_k[m] >> s;
-      if ((s_k[m + 1] >> s) == t) {
-        uint32_t b = m - 1;
-        while (b > 0 && m - b <= kShortRun && (s_k[b] >> s) == t) --b;
-        if ((s_k[b] >> s) != t) sort_run_serial<V, KV>(keys, vals, c0 + b, seg1, t, s, a.xf);
-      }
+    // This thread's keys of the list.
+    uint32_t move[PER];
+    V v[KV ? PER : 1];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t q = tid + (uint32_t)j * 256;
+      move[j] = q < count ? s_list[q] : 0;
+      if constexpr (KV)
+        if (move[j] >> 16 != (move[j] & 0xFFFFu)) v[j] = vals[c0 + (move[j] & 0xFFFFu)];
     }
-    __syncthreads();  // before the next chunk's first key is read and the list is reused
+    __syncthreads();  // every payload that moves is read
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t i = move[j] & 0xFFFFu, dst = move[j] >> 16;
+      if (dst == i) continue;
+      keys[c0 + dst] = from_ordered(at(i), a.xf);
+      if constexpr (KV) vals[c0 + dst] = v[j];
+    }
+    lds_barrier();  // the chunk's keys are read
   }
 }
 
